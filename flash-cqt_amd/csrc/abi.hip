@@ -58,30 +58,8 @@ extern "C" int fcqt_analysis(const fcqt_tables* tab, const int32_t* route, const
     // validate the band half before launching the FFT half
     if (int e = check_band_args(tab, route, coef_re, coef_im, layout, batch)) return e;
     if (!aligned(xs, 8)) return FCQT_EALIGN;
-    if (batch < kAnalysisChunkMinBatch) {
-        if (int e = fcqt_packed_fft_fwd(tab, x, xs, work, batch, stream)) return e;
-        return fcqt_route_bands(tab, route, xs, coef_re, coef_im, layout, batch, stream);
-    }
-    // Large batches run in chunks of kAnalysisChunk slices, all three
-    // kernels per chunk, so that a chunk's W and X (0.5 MB per slice) are
-    // still in the memory-side cache when its row pass and route read them;
-    // over a whole large batch they are not, and the route's gathers wait on
-    // HBM. One call against chunks of 128 (stream launches, hipEvents):
-    // B = 256 145 against 135 us, 384 261 against 208, 512 372 against 272,
-    // 1024 700 against 553; at B = 192 one call was faster (95-97 against
-    // 115 us). Slices are independent and every batch form gives the same
-    // bits, so the results do not depend on the chunking.
-    const int64_t cstride = layout == FCQT_PLANAR ? tab->ncoef : 2 * tab->ncoef;   // floats per coefficient row
-    for (int64_t lo = 0; lo < batch; lo += kAnalysisChunk) {
-        const int64_t n = batch - lo < kAnalysisChunk ? batch - lo : kAnalysisChunk;
-        float* xs_c = xs + lo * 2 * (int64_t)kXStride;
-        if (int e = fcqt_packed_fft_fwd(tab, x + lo * (int64_t)kN, xs_c, work + lo * 2 * (int64_t)kL, n, stream))
-            return e;
-        if (int e = fcqt_route_bands(tab, route, xs_c, coef_re + lo * cstride,
-                                     layout == FCQT_PLANAR ? coef_im + lo * cstride : coef_im, layout, n, stream))
-            return e;
-    }
-    return FCQT_OK;
+    if (int e = fcqt_packed_fft_fwd(tab, x, xs, work, batch, stream)) return e;
+    return fcqt_route_bands(tab, route, xs, coef_re, coef_im, layout, batch, stream);
 }
 
 extern "C" int fcqt_synthesis(const fcqt_tables* tab, const int32_t* scat, const int32_t* ovf,
@@ -93,7 +71,7 @@ extern "C" int fcqt_synthesis(const fcqt_tables* tab, const int32_t* scat, const
     if (!tab || !tab->tw_pass || !tab->tw_half || batch < 1 || batch > kMaxBatch) return FCQT_EARG;
     if (!aligned(f, 16) || !aligned(y, 8) || !aligned(work, 8) || !aligned(ovf, 4)) return FCQT_EALIGN;
     if (int e = fcqt_scatter_bands(tab, scat, coef_re, coef_im, layout, f, batch, stream)) return e;
-    return fcqt_packed_fft_inv(tab, ovf, f, y, work, batch, stream);
+    return packed_fft_inv(tab, ovf, f, y, work, batch, true, stream);
 }
 
 extern "C" int fcqt_stream_synthesis(const fcqt_tables* tab, const int32_t* scat, const int32_t* groups,

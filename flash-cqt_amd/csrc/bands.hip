@@ -37,7 +37,7 @@
 
 namespace fcqt {
 
-template <int LAYOUT, bool WT, bool SM>
+template <int LAYOUT, Store S, bool SM>
 __global__ __launch_bounds__(kBandThreads) void k_route_bands(const float2* __restrict__ xs,
                                                               float* __restrict__ cre,
                                                               float* __restrict__ cim,
@@ -49,10 +49,10 @@ __global__ __launch_bounds__(kBandThreads) void k_route_bands(const float2* __re
     __shared__ float2 lds[kBandTaskLds];
     int task_id, b;
     decode_task<false, SM>(batch, ntasks, task_id, b);
-    route_task<LAYOUT, WT>(task_id, b, xs, cre, cim, rec, tasks, ncoef, sm, tws, lds);
+    route_task<LAYOUT, S>(task_id, b, xs, cre, cim, rec, tasks, ncoef, sm, tws, lds);
 }
 
-template <int LAYOUT, bool WT, bool SM>
+template <int LAYOUT, Store S, bool SM, bool STREAM = false>
 __global__ __launch_bounds__(kBandThreads) void k_scatter_bands(const float* __restrict__ cre,
                                                                 const float* __restrict__ cim,
                                                                 float* __restrict__ f,
@@ -64,7 +64,7 @@ __global__ __launch_bounds__(kBandThreads) void k_scatter_bands(const float* __r
     __shared__ float2 lds[kBandTaskLds];
     int task_id, b;
     decode_task<true, SM>(batch, ntasks, task_id, b);
-    scatter_task<LAYOUT, WT>(task_id, b, cre, cim, f, scat, tasks, ncoef, sm, tws, lds);
+    scatter_task<LAYOUT, S, STREAM>(task_id, b, cre, cim, f, scat, tasks, ncoef, sm, tws, lds);
 }
 
 // From this batch size on the band kernels write their outputs through the
@@ -87,26 +87,30 @@ constexpr int64_t kBandWriteThroughMaxBatch = 104;
 // against 36.9 us). Same results either way.
 constexpr int64_t kBandSliceMajorMinBatch = 64;
 
+// total: slices of the whole call that this batch is a chunk of.
 template <int LAYOUT>
 static void launch_route(int64_t ntasks, int64_t batch, hipStream_t stream, const float2* xs, float* cre,
                          float* cim, const int2* rec, const int4* tasks, long ncoef, const SliceMap& sm,
-                         const float2* tws) {
+                         const float2* tws, int64_t total) {
     const dim3 grid((unsigned)(ntasks * batch));
     static_assert(kBandWriteThroughMinBatch <= kBandSliceMajorMinBatch &&
                       kBandSliceMajorMinBatch <= kBandWriteThroughMaxBatch,
                   "batch ranges: plain task-major, write-through task-major, write-through slice-major, "
                   "plain slice-major");
-    if (batch > kBandWriteThroughMaxBatch)
-        hipLaunchKernelGGL((k_route_bands<LAYOUT, false, true>), grid, dim3(kBandThreads), 0, stream, xs, cre, cim,
+    if (total >= (LAYOUT == kSliced ? kStreamSlicedCoefMinBatch : kStreamCoefOutMinBatch))
+        hipLaunchKernelGGL((k_route_bands<LAYOUT, Store::kStream, true>), grid, dim3(kBandThreads), 0, stream, xs, cre,
+                           cim, rec, tasks, (int)batch, ncoef, sm, tws, (int)ntasks);
+    else if (batch > kBandWriteThroughMaxBatch)
+        hipLaunchKernelGGL((k_route_bands<LAYOUT, Store::kPlain, true>), grid, dim3(kBandThreads), 0, stream, xs, cre, cim,
                            rec, tasks, (int)batch, ncoef, sm, tws, (int)ntasks);
     else if (batch >= kBandSliceMajorMinBatch)
-        hipLaunchKernelGGL((k_route_bands<LAYOUT, true, true>), grid, dim3(kBandThreads), 0, stream, xs, cre, cim,
+        hipLaunchKernelGGL((k_route_bands<LAYOUT, Store::kThrough, true>), grid, dim3(kBandThreads), 0, stream, xs, cre, cim,
                            rec, tasks, (int)batch, ncoef, sm, tws, (int)ntasks);
     else if (batch >= kBandWriteThroughMinBatch)
-        hipLaunchKernelGGL((k_route_bands<LAYOUT, true, false>), grid, dim3(kBandThreads), 0, stream, xs, cre, cim,
+        hipLaunchKernelGGL((k_route_bands<LAYOUT, Store::kThrough, false>), grid, dim3(kBandThreads), 0, stream, xs, cre, cim,
                            rec, tasks, (int)batch, ncoef, sm, tws, (int)ntasks);
     else
-        hipLaunchKernelGGL((k_route_bands<LAYOUT, false, false>), grid, dim3(kBandThreads), 0, stream, xs, cre, cim,
+        hipLaunchKernelGGL((k_route_bands<LAYOUT, Store::kPlain, false>), grid, dim3(kBandThreads), 0, stream, xs, cre, cim,
                            rec, tasks, (int)batch, ncoef, sm, tws, (int)ntasks);
 }
 
@@ -115,17 +119,20 @@ static void launch_scatter(int64_t ntasks, int64_t batch, hipStream_t stream, co
                            float* f, const int2* scat, const int4* tasks, long ncoef, const SliceMap& sm,
                            const float2* tws) {
     const dim3 grid((unsigned)(ntasks * batch));
-    if (batch > kBandWriteThroughMaxBatch)
-        hipLaunchKernelGGL((k_scatter_bands<LAYOUT, false, true>), grid, dim3(kBandThreads), 0, stream, cre, cim, f,
+    if (batch >= (LAYOUT == kSliced ? kStreamSlicedCoefMinBatch : kStreamCoefInMinBatch))
+        hipLaunchKernelGGL((k_scatter_bands<LAYOUT, Store::kPlain, true, true>), grid, dim3(kBandThreads), 0, stream,
+                           cre, cim, f, scat, tasks, (int)batch, ncoef, sm, tws, (int)ntasks);
+    else if (batch > kBandWriteThroughMaxBatch)
+        hipLaunchKernelGGL((k_scatter_bands<LAYOUT, Store::kPlain, true>), grid, dim3(kBandThreads), 0, stream, cre, cim, f,
                            scat, tasks, (int)batch, ncoef, sm, tws, (int)ntasks);
     else if (batch >= kBandSliceMajorMinBatch)
-        hipLaunchKernelGGL((k_scatter_bands<LAYOUT, true, true>), grid, dim3(kBandThreads), 0, stream, cre, cim, f,
+        hipLaunchKernelGGL((k_scatter_bands<LAYOUT, Store::kThrough, true>), grid, dim3(kBandThreads), 0, stream, cre, cim, f,
                            scat, tasks, (int)batch, ncoef, sm, tws, (int)ntasks);
     else if (batch >= kBandWriteThroughMinBatch)
-        hipLaunchKernelGGL((k_scatter_bands<LAYOUT, true, false>), grid, dim3(kBandThreads), 0, stream, cre, cim, f,
+        hipLaunchKernelGGL((k_scatter_bands<LAYOUT, Store::kThrough, false>), grid, dim3(kBandThreads), 0, stream, cre, cim, f,
                            scat, tasks, (int)batch, ncoef, sm, tws, (int)ntasks);
     else
-        hipLaunchKernelGGL((k_scatter_bands<LAYOUT, false, false>), grid, dim3(kBandThreads), 0, stream, cre, cim, f,
+        hipLaunchKernelGGL((k_scatter_bands<LAYOUT, Store::kPlain, false>), grid, dim3(kBandThreads), 0, stream, cre, cim, f,
                            scat, tasks, (int)batch, ncoef, sm, tws, (int)ntasks);
 }
 
@@ -161,10 +168,10 @@ extern "C" int fcqt_route_bands(const fcqt_tables* tab, const int32_t* route, co
     const auto* ws = reinterpret_cast<const float2*>(tab->tw_stage);
     if (layout == FCQT_PLANAR)
         launch_route<FCQT_PLANAR>(tab->ntasks, batch, stream, xx, coef_re, coef_im, rr, tt, (long)tab->ncoef,
-                                  SliceMap{nullptr, 1, 0}, ws);
+                                  SliceMap{nullptr, 1, 0}, ws, batch);
     else
         launch_route<FCQT_INTERLEAVED>(tab->ntasks, batch, stream, xx, coef_re, coef_re, rr, tt, (long)tab->ncoef,
-                                       SliceMap{nullptr, 1, 0}, ws);
+                                       SliceMap{nullptr, 1, 0}, ws, batch);
     return launch_status();
 }
 
@@ -200,7 +207,7 @@ extern "C" int fcqt_route_bands_sliced(const fcqt_tables* tab, const int32_t* ro
                           (long)tab->ncoef,
                           SliceMap{reinterpret_cast<const int4*>(groups), (int)nslices, (int)first, (long)batch,
                                    (int)nslices, 0, 0},
-                          reinterpret_cast<const float2*>(tab->tw_stage));
+                          reinterpret_cast<const float2*>(tab->tw_stage), batch);
     return launch_status();
 }
 
@@ -218,8 +225,7 @@ extern "C" int fcqt_sliced_analysis(const fcqt_tables* tab, const int32_t* route
     // From kAnalysisChunkMinBatch slices on, chunks of about kAnalysisChunk
     // slices (all signals of a range of slices, or ranges of signals one
     // slice each), each framed, transformed and routed in turn so that its
-    // W and X are still in the memory-side cache when read (as fcqt_analysis
-    // does); a chunk's slices land in the whole call's block layout. The
+    // W and X are still in the memory-side cache when read; a chunk's slices land in the whole call's block layout. The
     // chunks reuse the leading rows of xs and work. Every slice gives the
     // same bits however the call is cut.
     int64_t ns = nsig, cs = nslices;
@@ -233,13 +239,13 @@ extern "C" int fcqt_sliced_analysis(const fcqt_tables* tab, const int32_t* route
         const int64_t na = nsig - a < ns ? nsig - a : ns;
         for (int64_t c = 0; c < nslices; c += cs) {
             const int64_t nc = nslices - c < cs ? nslices - c : cs;
-            if (int e = fcqt_slice_fft_fwd(tab, sig + a * sig_len, sig_len, window, na, nc, c, 0, xs, work, stream))
+            if (int e = slice_fft_fwd(tab, sig + a * sig_len, sig_len, window, na, nc, c, 0, xs, work, batch, stream))
                 return e;
             launch_route<kSliced>(tab->ntasks, na * nc, stream, reinterpret_cast<const float2*>(xs), coef, coef,
                                   reinterpret_cast<const int2*>(route), reinterpret_cast<const int4*>(tab->tasks),
                                   (long)tab->ncoef,
                                   SliceMap{g4, (int)nc, (int)c, (long)batch, (int)nslices, (int)c, (int)a},
-                                  reinterpret_cast<const float2*>(tab->tw_stage));
+                                  reinterpret_cast<const float2*>(tab->tw_stage), batch);
             if (int e = launch_status()) return e;
         }
     }

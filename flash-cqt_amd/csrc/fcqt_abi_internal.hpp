@@ -14,11 +14,40 @@ namespace fcqt {
 // kernel has the most workgroups per slice (< 256), so this is generous.
 constexpr int64_t kMaxBatch = 1 << 22;
 
-// fcqt_analysis runs batches of kAnalysisChunkMinBatch slices and more in
-// chunks of kAnalysisChunk (the measurements are at the loop in abi.hip)
+// fcqt_sliced_analysis runs calls of kAnalysisChunkMinBatch slices and more
+// in chunks of about kAnalysisChunk (the header's buffer contract)
 constexpr int64_t kAnalysisChunk = FCQT_ANALYSIS_CHUNK;
 constexpr int64_t kAnalysisChunkMinBatch = FCQT_ANALYSIS_CHUNK_MIN_BATCH;
 static_assert(kAnalysisChunk == 128 && kAnalysisChunkMinBatch == 256, "chunk constants of the header");
+
+// From these batch sizes on a buffer is written or read past the caches
+// (Store::kStream, load_in<true>). Per slice a round trip touches x, W, X,
+// the coefficients, F and y: 2.7 MB, so about 96 slices fill the 256 MB
+// memory-side cache, and past that a buffer without a nearby reader only
+// pushes W, X and F out to HBM. Measured as loops over three inputs, kept in
+// the caches against streamed (us, headline layout; round trip, or the
+// direction that is named):
+//   x:      B = 96 104.4 / 96.7, 127 140.8 / 133.3, but the analysis alone
+//           112 53.5 / 56.2, 120 58.2 / 59.3, 127 62.2 / 62.4, 160 80.1 / 75.0
+//   y:      B = 105 116.2 / 113.5, 127 140.8 / 137.8, 144 165.6 / 162.9 (with x)
+//   coefficients read by the scatter (with x, y): B = 127 130.5 / 138.9,
+//           136 147.9 / 149.6, 144 162.9 / 153.7, 160 189.5 / 166.8
+//   coefficients written by the route (with those): B = 160 166.8 / 167.2,
+//           176 183.9 / 182.8, 200 210.3 / 206.4, 512 592 / 550; the analysis
+//           alone 256 134.7 / 117.4, 512 271.8 / 221.2
+//   W read by the row pass (with those): B = 192 194.7 / 194.9,
+//           256 266.1 / 257.7, 512 550 / 518
+// SlicedCQT's coefficients go to a new buffer each call, and streaming both
+// their ends pays earlier: 120 slices 144.4 / 139.2, 128 153.6 / 145.1, 160
+// 212.9 / 188.9, 224 296.4 / 262.3 (its analysis alone 57.6 / 58.6 at 120,
+// 116.2 / 100.9 at 224); its signals are read twice (the overlap) and its
+// slice buffer is read again by the overlap-add, so those are not streamed.
+constexpr int64_t kStreamXMinBatch = 124;
+constexpr int64_t kStreamYMinBatch = 105;
+constexpr int64_t kStreamCoefInMinBatch = 140;
+constexpr int64_t kStreamCoefOutMinBatch = 192;
+constexpr int64_t kStreamWMinBatch = 192;
+constexpr int64_t kStreamSlicedCoefMinBatch = 105;
 
 inline bool aligned(const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
 
@@ -27,6 +56,18 @@ inline bool aligned(const void* p, uintptr_t a) { return (reinterpret_cast<uintp
 // layout, alignment; defined in bands.hip.
 int check_band_args(const fcqt_tables* tab, const int32_t* rec, const float* cre, const float* cim, int layout,
                     int64_t batch);
+
+// fcqt_packed_fft_inv; last = true when nothing reads y soon after the call
+// (large batches then store it without keeping it in the caches); defined
+// in packed_fft.hip.
+int packed_fft_inv(const fcqt_tables* tab, const int32_t* ovf, const float* f, float* y, float* work, int64_t batch,
+                   bool last, hipStream_t stream);
+
+// fcqt_slice_fft_fwd of one chunk of a call of `total` slices (which sets
+// the cache choices); defined in packed_fft.hip.
+int slice_fft_fwd(const fcqt_tables* tab, const float* sig, int64_t sig_len, const float* window, int64_t nsig,
+                  int64_t nslices, int64_t first, int64_t origin, float* xs, float* work, int64_t total,
+                  hipStream_t stream);
 
 // Text of the last failed launch on this host thread.
 inline char* last_error_buf() {

@@ -75,19 +75,19 @@ __device__ __forceinline__ void unit_coef(const int4 task, const int task_id, co
     }
 }
 
-template <int LAYOUT>
+template <int LAYOUT, bool STREAM>
 __device__ __forceinline__ float2 load_coef(const float* __restrict__ cre, const float* __restrict__ cim, int i) {
-    if constexpr (LAYOUT == FCQT_PLANAR) return make_float2(cre[i], cim[i]);
-    else return reinterpret_cast<const float2*>(cre)[i];
+    if constexpr (LAYOUT == FCQT_PLANAR) return make_float2(load_in<STREAM>(cre + i), load_in<STREAM>(cim + i));
+    else return load_in<STREAM>(reinterpret_cast<const float2*>(cre) + i);
 }
 
-template <int LAYOUT, bool WT>
+template <int LAYOUT, Store S>
 __device__ __forceinline__ void store_coef(float* __restrict__ cre, float* __restrict__ cim, int i, float2 v) {
     if constexpr (LAYOUT == FCQT_PLANAR) {
-        store_out<WT>(cre + i, v.x);
-        store_out<WT>(cim + i, v.y);
+        store_out<S>(cre + i, v.x);
+        store_out<S>(cim + i, v.y);
     } else {
-        store_out<WT>(reinterpret_cast<float2*>(cre) + i, v);
+        store_out<S>(reinterpret_cast<float2*>(cre) + i, v);
     }
 }
 
@@ -102,7 +102,7 @@ __device__ __forceinline__ void load_records(int2* rv, const int2* __restrict__ 
 // task's bands (units past the band count compute padding that is never
 // stored). The twiddle loads issue before the gathers, so their latency
 // hides under the record and gather round trips.
-template <int M, int LAYOUT, bool WT>
+template <int M, int LAYOUT, Store S>
 __device__ __forceinline__ void route_band(const int4 task, const int task_id, const int b,
                                            const int2* rv, const float2* __restrict__ xb,
                                            float* __restrict__ cre, float* __restrict__ cim,
@@ -138,12 +138,12 @@ __device__ __forceinline__ void route_band(const int4 task, const int task_id, c
         for (int q = 0; q < P::QL; ++q) {
 #pragma unroll
             for (int r = 0; r < P::RL; ++r)
-                store_coef<LAYOUT, WT>(orow, oim, (t + P::T * q + r * P::OS + shift) & (M - 1), v[q * P::RL + r]);
+                store_coef<LAYOUT, S>(orow, oim, (t + P::T * q + r * P::OS + shift) & (M - 1), v[q * P::RL + r]);
         }
     }
 }
 
-template <int M, int LAYOUT, bool WT>
+template <int M, int LAYOUT, Store S, bool STREAM>
 __device__ __forceinline__ void scatter_band(const int4 task, const int task_id, const int b,
                                              const int2* __restrict__ scat, const float* __restrict__ cre,
                                              const float* __restrict__ cim, float* __restrict__ f,
@@ -163,7 +163,7 @@ __device__ __forceinline__ void scatter_band(const int4 task, const int task_id,
     const float* ci = cim + (LAYOUT == FCQT_PLANAR ? ib : 0);
     float2 v[16];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) v[r] = load_coef<LAYOUT>(cr, ci, (t + P::T * r + shift) & (M - 1));
+    for (int r = 0; r < 16; ++r) v[r] = load_coef<LAYOUT, STREAM>(cr, ci, (t + P::T * r + shift) & (M - 1));
     Tw2Copy<M, kBandThreads> c2;
     fetch_tw2<M, kBandThreads>(c2, tws, tid);
     Tw3<M> w3;
@@ -181,7 +181,7 @@ __device__ __forceinline__ void scatter_band(const int4 task, const int task_id,
                 const unsigned mode = (unsigned)rv[i].x >> 30;
                 const unsigned slot = min((unsigned)rv[i].x & 0x3fffffffu, (unsigned)(kFRow - 1));
                 const float gi = mode == 0 ? gr : (mode == 1 ? -gr : 0.0f);
-                store_out<WT>(fb + slot, make_float2(gr * v[i].x, gi * v[i].y));
+                store_out<S>(fb + slot, make_float2(gr * v[i].x, gi * v[i].y));
             }
         }
     }
@@ -205,9 +205,8 @@ constexpr int kBandTaskLds = kBandLds + tw2_len<2048>();
 
 // One band task (task_id, slice b) of the route engine in caller-provided
 // LDS; the band kernels and the single-launch analysis (persist.hip) run it.
-// WT: write the coefficients through the L2 (store_out), for batches whose
-// coefficient output is large.
-template <int LAYOUT, bool WT = false>
+// S: how the coefficients are stored (store_out).
+template <int LAYOUT, Store S = Store::kPlain>
 __device__ __forceinline__ void route_task(const int task_id, const int b, const float2* __restrict__ xs,
                                            float* __restrict__ cre, float* __restrict__ cim,
                                            const int2* __restrict__ rec, const int4* __restrict__ tasks,
@@ -222,7 +221,7 @@ __device__ __forceinline__ void route_task(const int task_id, const int b, const
     const float2* xb = xs + (long)b * kXStride;
     const int4 td = tasks[task_id];
     if (td.y < 0 || (long)td.y + (long)td.z * td.x > ncoef) return;   // task outside the coefficient row
-#define FCQT_ROUTE(M_) route_band<M_, LAYOUT, WT>(td, task_id, b, rv, xb, cre, cim, ncoef, sm, tws, lds, tw2, tid)
+#define FCQT_ROUTE(M_) route_band<M_, LAYOUT, S>(td, task_id, b, rv, xb, cre, cim, ncoef, sm, tws, lds, tw2, tid)
     switch (td.x) {
         case 32: FCQT_ROUTE(32); break;
         case 64: FCQT_ROUTE(64); break;
@@ -237,9 +236,10 @@ __device__ __forceinline__ void route_task(const int task_id, const int b, const
 }
 
 
-// One band task of the scatter engine in caller-provided LDS (WT: slot
-// stores through the L2, as in route_task).
-template <int LAYOUT, bool WT = false>
+// One band task of the scatter engine in caller-provided LDS (S: how the
+// slots are stored; STREAM: coefficients read without keeping them in the
+// caches).
+template <int LAYOUT, Store S = Store::kPlain, bool STREAM = false>
 __device__ __forceinline__ void scatter_task(const int task_id, const int b, const float* __restrict__ cre,
                                              const float* __restrict__ cim, float* __restrict__ f,
                                              const int2* __restrict__ scat, const int4* __restrict__ tasks,
@@ -249,7 +249,7 @@ __device__ __forceinline__ void scatter_task(const int task_id, const int b, con
     float2* tw2 = lds + kBandLds;
     const int4 td = tasks[task_id];
     if (td.y < 0 || (long)td.y + (long)td.z * td.x > ncoef) return;   // task outside the coefficient row
-#define FCQT_SCATTER(M_) scatter_band<M_, LAYOUT, WT>(td, task_id, b, scat, cre, cim, f, ncoef, sm, tws, lds, tw2, tid)
+#define FCQT_SCATTER(M_) scatter_band<M_, LAYOUT, S, STREAM>(td, task_id, b, scat, cre, cim, f, ncoef, sm, tws, lds, tw2, tid)
     switch (td.x) {
         case 32: FCQT_SCATTER(32); break;
         case 64: FCQT_SCATTER(64); break;

@@ -49,8 +49,8 @@ __device__ __forceinline__ float2 cmul(float2 a, float2 b) {
 __device__ __forceinline__ float2 cmulc(float2 a, float2 b) {
     return make_float2(fmaf(a.x, b.x, a.y * b.y), fmaf(a.y, b.x, -a.x * b.y));
 }
-// ------------------------------------------------------------ output stores
-// WT = true: a store that writes through this XCD's L2 (a relaxed device-scope
+// ------------------------------------------- output stores, streamed loads
+// kThrough: a store that writes through this XCD's L2 (a relaxed device-scope
 // atomic store, 'sc1'), so the line goes on to the memory-side cache at once
 // instead of staying dirty in the L2 until the write-back at the end of the
 // kernel, which then no longer sits on the critical path. It pays for
@@ -58,11 +58,22 @@ __device__ __forceinline__ float2 cmulc(float2 a, float2 b) {
 // are final): the band kernels from 4 slices up and the wide inverse
 // passes. A line written this way is not kept in the writer's L2, so a
 // consumer on the same XCD no longer hits it there, and a store covering
-// half a 128-byte line costs extra bytes. The values stored are the same
-// either way.
-template <bool WT>
+// half a 128-byte line costs extra bytes.
+// kStream: a non-temporal store, which leaves no copy in the caches. It pays
+// for outputs that fall out of the 256 MB memory-side cache before anything
+// reads them anyway, because the intermediates then stay there.
+// load_in<true> is the same for inputs read once. The values are the same
+// with every form.
+enum class Store { kPlain, kThrough, kStream };
+
+typedef float vec2f __attribute__((ext_vector_type(2)));
+
+template <Store S>
 __device__ __forceinline__ void store_out(float2* p, float2 v) {
-    if constexpr (WT) {
+    if constexpr (S == Store::kStream) {
+        const vec2f a = {v.x, v.y};
+        __builtin_nontemporal_store(a, reinterpret_cast<vec2f*>(p));
+    } else if constexpr (S == Store::kThrough) {
         const unsigned long long bits =
             ((unsigned long long)__float_as_uint(v.y) << 32) | (unsigned long long)__float_as_uint(v.x);
         __hip_atomic_store(reinterpret_cast<unsigned long long*>(p), bits, __ATOMIC_RELAXED,
@@ -71,13 +82,30 @@ __device__ __forceinline__ void store_out(float2* p, float2 v) {
         *p = v;
     }
 }
-template <bool WT>
+template <Store S>
 __device__ __forceinline__ void store_out(float* p, float v) {
-    if constexpr (WT)
+    if constexpr (S == Store::kStream)
+        __builtin_nontemporal_store(v, p);
+    else if constexpr (S == Store::kThrough)
         __hip_atomic_store(reinterpret_cast<unsigned*>(p), __float_as_uint(v), __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_AGENT);
     else
         *p = v;
+}
+
+template <bool STREAM>
+__device__ __forceinline__ float2 load_in(const float2* p) {
+    if constexpr (STREAM) {
+        const vec2f a = __builtin_nontemporal_load(reinterpret_cast<const vec2f*>(p));
+        return make_float2(a.x, a.y);
+    } else {
+        return *p;
+    }
+}
+template <bool STREAM>
+__device__ __forceinline__ float load_in(const float* p) {
+    if constexpr (STREAM) return __builtin_nontemporal_load(p);
+    else return *p;
 }
 
 // a * (SIGN i)   i.e. a * e^{SIGN i pi/2}

@@ -108,9 +108,11 @@ __device__ __forceinline__ float2 sliced_pair_vec(const SliceSrc& src, const Sli
 // Each pass is a tile body over (slice b, tile index) working in LDS the
 // caller provides (the kernels below and the single-launch kernels of
 // persist.hip run the same bodies, so both give the same bits): CPW (or RPW)
-// units, then the twiddle block. The inverse passes take WT, the store form:
-// the wide shapes write through the L2 up to kInvWriteThroughMaxBatch slices
-// (store_out<true>: the inverse pair ran 1.4 us faster at batch 64) and plainly
+// units, then the twiddle block. S is the store form, STREAM the load form of
+// the input (fcqt_abi_internal.hpp says from which batch sizes on buffers
+// bypass the caches). The inverse passes' wide shapes
+// write through the L2 up to kInvWriteThroughMaxBatch slices
+// (Store::kThrough: the inverse pair ran 1.4 us faster at batch 64) and plainly
 // above, where the round trip's working set outgrows the memory-side cache
 // (round trips 119.4-119.8 against 120.6-121.1 us at B = 112, 142.9-143.1
 // against 145.9 us at B = 128, 308.4-308.6 against 314.0 us at B = 256; 101
@@ -126,7 +128,7 @@ constexpr int col_lds() { return CPW * Plan<128>::US + tw2_len<128>(); }
 template <int RPW>
 constexpr int row_lds() { return RPW * Plan<256>::US + tw2_len<256>(); }
 
-template <bool SLICED, int CPW>
+template <bool SLICED, int CPW, bool STREAM = false>
 __device__ __forceinline__ void col_fwd_tile(const int b, const int cg, const float2* __restrict__ in,
                                              float2* __restrict__ out, const float2* __restrict__ twp,
                                              const float2* __restrict__ tws, const SliceSrc& src, float2* lds,
@@ -156,7 +158,7 @@ __device__ __forceinline__ void col_fwd_tile(const int b, const int cg, const fl
     } else {
         const float2* xb = in + (long)b * kL;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) v[r] = xb[256 * (t + 8 * r) + n2];
+        for (int r = 0; r < 16; ++r) v[r] = load_in<STREAM>(xb + 256 * (t + 8 * r) + n2);
     }
     // every twiddle this thread needs, in flight with the data
     load_tw2_lds<128>(tw2, tws, tid, 8 * CPW);
@@ -200,7 +202,7 @@ __device__ __forceinline__ int inv_col(int w, int c) {
     return c < H ? p : (p == 0 ? 128 : 256 - p);
 }
 
-template <int CPW, bool WT>
+template <int CPW, Store S>
 __device__ __forceinline__ void col_inv_tile(const int b, const int w, const float2* __restrict__ f,
                                              float2* __restrict__ out, const float2* __restrict__ twp,
                                              const float2* __restrict__ twn, const int* __restrict__ fold,
@@ -318,7 +320,7 @@ __device__ __forceinline__ void col_inv_tile(const int b, const int w, const flo
 #pragma unroll
         for (int r = 0; r < P::RL; ++r) {
             const int k1 = t + 8 * q + 16 * r;
-            store_out<WT>(&yb[k1 * 256 + col], cmul(v[q * P::RL + r], tp[q * P::RL + r]));
+            store_out<S>(&yb[k1 * 256 + col], cmul(v[q * P::RL + r], tp[q * P::RL + r]));
         }
     }
 }
@@ -342,14 +344,14 @@ __device__ __forceinline__ int fwd_row(int w, int rho) {
 // vhold / shold: a per-thread value and 16 workgroup-uniform values loaded
 // before the call that must arrive with the row data (the untangle
 // twiddles), so their loads are not deferred past the barriers.
-template <bool HOLD>
+template <bool HOLD, bool STREAM>
 __device__ __forceinline__ void row_fft_to_lds(const float2* __restrict__ yrow, float2* lds, float2* tw2,
                                                int rho, int t, int nthreads, const float2* __restrict__ tws,
                                                float2* vhold, float2* shold, const int tid) {
     using P = Plan<256>;
     float2 v[16];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) v[r] = yrow[t + 16 * r];
+    for (int r = 0; r < 16; ++r) v[r] = load_in<STREAM>(yrow + t + 16 * r);
     load_tw2_lds<256>(tw2, tws, tid, nthreads);
     if constexpr (HOLD) {
         asm volatile("" : "+v"(vhold->x), "+v"(vhold->y));
@@ -370,7 +372,7 @@ __device__ __forceinline__ void row_fft_to_lds(const float2* __restrict__ yrow, 
     __syncthreads();
 }
 
-template <int RPW>
+template <int RPW, bool STREAM = false>
 __device__ __forceinline__ void row_fwd_tile(const int b, const int w, const float2* __restrict__ in,
                                              float2* __restrict__ xs, const float2* __restrict__ twn,
                                              const float2* __restrict__ tws, float2* lds,
@@ -389,7 +391,7 @@ __device__ __forceinline__ void row_fwd_tile(const int b, const int w, const flo
     float2 wu[16];
 #pragma unroll
     for (int u = 0; u < 16; ++u) wu[u] = twn[2048 * u];
-    row_fft_to_lds<true>(in + (long)b * kL + (long)fwd_row<RPW>(w, rho) * 256, lds, tw2, rho, t, 16 * RPW, tws,
+    row_fft_to_lds<true, STREAM>(in + (long)b * kL + (long)fwd_row<RPW>(w, rho) * 256, lds, tw2, rho, t, 16 * RPW, tws,
                          &wb, wu, tid);
     // untangle: lanes walk the tile's rows for coalesced stores
     const float2* s = lds + rho2 * P::US;
@@ -417,7 +419,7 @@ __device__ __forceinline__ void row_fwd_tile(const int b, const int w, const flo
 }
 
 
-template <int RPW, bool WT>
+template <int RPW, Store S, bool STREAM = false>
 __device__ __forceinline__ void row_inv_tile(const int b, const int rg, const float2* __restrict__ in,
                                              float2* __restrict__ y, const float2* __restrict__ tws, float2* lds,
                                              const int tid = threadIdx.x) {
@@ -425,7 +427,7 @@ __device__ __forceinline__ void row_inv_tile(const int b, const int rg, const fl
     float2* tw2 = lds + RPW * P::US;
     const int rho = tid >> 4;
     const int t = tid & 15;
-    row_fft_to_lds<false>(in + (long)b * kL + (long)(rg * RPW + rho) * 256, lds, tw2, rho, t, 16 * RPW, tws,
+    row_fft_to_lds<false, STREAM>(in + (long)b * kL + (long)(rg * RPW + rho) * 256, lds, tw2, rho, t, 16 * RPW, tws,
                           nullptr, nullptr, tid);
     const int rho2 = tid & (RPW - 1);
     const int kg = tid / RPW;
@@ -437,7 +439,7 @@ __device__ __forceinline__ void row_inv_tile(const int b, const int rg, const fl
     for (int u = 0; u < 16; ++u) {
         const int k2 = kg + 16 * u;
         const float2 w = s2[pad16(k2)];
-        store_out<WT>(&yo[kk1 + 128 * k2], make_float2(w.x * sc, -w.y * sc));
+        store_out<S>(&yo[kk1 + 128 * k2], make_float2(w.x * sc, -w.y * sc));
     }
 }
 
@@ -461,7 +463,7 @@ __device__ __forceinline__ void row_inv_ola_tile(const int b, const int rg, cons
     float2* tw2 = lds + RPW * P::US;
     const int rho = tid >> 4;
     const int t = tid & 15;
-    row_fft_to_lds<false>(in + (long)b * kL + (long)(rg * RPW + rho) * 256, lds, tw2, rho, t, 16 * RPW, tws,
+    row_fft_to_lds<false, false>(in + (long)b * kL + (long)(rg * RPW + rho) * 256, lds, tw2, rho, t, 16 * RPW, tws,
                           nullptr, nullptr, tid);
     const int rho2 = tid & (RPW - 1);
     const int kg = tid / RPW;

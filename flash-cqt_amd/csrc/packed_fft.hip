@@ -29,7 +29,7 @@
 
 namespace fcqt {
 
-template <bool SLICED, int CPW>
+template <bool SLICED, int CPW, bool STREAM = false>
 __global__ __launch_bounds__(8 * CPW) void k_col_fwd(const float2* __restrict__ in, float2* __restrict__ out,
                                                      const float2* __restrict__ twp,
                                                      const float2* __restrict__ tws, const SliceSrc src) {
@@ -37,10 +37,10 @@ __global__ __launch_bounds__(8 * CPW) void k_col_fwd(const float2* __restrict__ 
     __shared__ float2 lds[col_lds<CPW>()];
     const int lg = xcd_remap((int)blockIdx.x, (int)gridDim.x);
     const int b = lg / kWgs;
-    col_fwd_tile<SLICED, CPW>(b, lg - b * kWgs, in, out, twp, tws, src, lds);
+    col_fwd_tile<SLICED, CPW, STREAM>(b, lg - b * kWgs, in, out, twp, tws, src, lds);
 }
 
-template <int CPW, bool WT>
+template <int CPW, Store S>
 __global__ __launch_bounds__(8 * CPW) void k_col_inv(const float2* __restrict__ f, float2* __restrict__ out,
                                                      const float2* __restrict__ twp,
                                                      const float2* __restrict__ twn,
@@ -50,10 +50,10 @@ __global__ __launch_bounds__(8 * CPW) void k_col_inv(const float2* __restrict__ 
     __shared__ float2 lds[col_lds<CPW>()];
     const int lg = xcd_remap((int)blockIdx.x, (int)gridDim.x);
     const int b = lg / kWgs;
-    col_inv_tile<CPW, WT>(b, lg - b * kWgs, f, out, twp, twn, fold, tws, lds);
+    col_inv_tile<CPW, S>(b, lg - b * kWgs, f, out, twp, twn, fold, tws, lds);
 }
 
-template <int RPW>
+template <int RPW, bool STREAM = false>
 __global__ __launch_bounds__(16 * RPW) void k_row_fwd(const float2* __restrict__ in, float2* __restrict__ xs,
                                                       const float2* __restrict__ twn,
                                                       const float2* __restrict__ tws) {
@@ -61,22 +61,23 @@ __global__ __launch_bounds__(16 * RPW) void k_row_fwd(const float2* __restrict__
     __shared__ float2 lds[row_lds<RPW>()];
     const int lg = xcd_remap((int)blockIdx.x, (int)gridDim.x);
     const int b = lg / kWgs;
-    row_fwd_tile<RPW>(b, lg - b * kWgs, in, xs, twn, tws, lds);
+    row_fwd_tile<RPW, STREAM>(b, lg - b * kWgs, in, xs, twn, tws, lds);
 }
 
-template <int RPW, bool WT>
+template <int RPW, Store S>
 __global__ __launch_bounds__(16 * RPW) void k_row_inv(const float2* __restrict__ in, float2* __restrict__ y,
                                                       const float2* __restrict__ tws) {
     constexpr int kWgs = 128 / RPW;               // workgroups per slice
     __shared__ float2 lds[row_lds<RPW>()];
     const int lg = xcd_remap((int)blockIdx.x, (int)gridDim.x);
     const int b = lg / kWgs;
-    row_inv_tile<RPW, WT>(b, lg - b * kWgs, in, y, tws, lds);
+    row_inv_tile<RPW, S>(b, lg - b * kWgs, in, y, tws, lds);
 }
 
 // Launch helpers: the pass kernels of one direction in the tile shape the
 // batch size selects.
-template <int CPW, int RPW>
+// (STREAM_X: x read once, non-temporally; STREAM_W: so is W by the row pass).
+template <int CPW, int RPW, bool STREAM_X = false, bool STREAM_W = false>
 static int launch_fwd_passes(const float2* x, float2* work, float2* xs, const float2* twp, const float2* twh,
                              const float2* tws, const SliceSrc& src, bool sliced, int64_t batch,
                              hipStream_t stream) {
@@ -84,37 +85,48 @@ static int launch_fwd_passes(const float2* x, float2* work, float2* xs, const fl
     if (sliced)
         hipLaunchKernelGGL((k_col_fwd<true, CPW>), gc, dim3(8 * CPW), 0, stream, x, work, twp, tws, src);
     else
-        hipLaunchKernelGGL((k_col_fwd<false, CPW>), gc, dim3(8 * CPW), 0, stream, x, work, twp, tws, src);
+        hipLaunchKernelGGL((k_col_fwd<false, CPW, STREAM_X>), gc, dim3(8 * CPW), 0, stream, x, work, twp, tws, src);
     if (int e = launch_status()) return e;
-    hipLaunchKernelGGL((k_row_fwd<RPW>), gr, dim3(16 * RPW), 0, stream, work, xs, twh, tws);
+    hipLaunchKernelGGL((k_row_fwd<RPW, STREAM_W>), gr, dim3(16 * RPW), 0, stream, work, xs, twh, tws);
     return launch_status();
 }
 
+// total: slices of the whole call that this batch is a chunk of.
 static int fwd_passes(const float2* x, float2* work, float2* xs, const float2* twp, const float2* twh,
-                      const float2* tws, const SliceSrc& src, bool sliced, int64_t batch, hipStream_t stream) {
+                      const float2* tws, const SliceSrc& src, bool sliced, int64_t batch, int64_t total,
+                      hipStream_t stream) {
     if (batch <= kNarrowMaxBatch)
         return launch_fwd_passes<kColsNarrow, kRowsNarrow>(x, work, xs, twp, twh, tws, src, sliced, batch, stream);
+    if (total >= kStreamWMinBatch)
+        return launch_fwd_passes<kColsWide, kRowsWide, true, true>(x, work, xs, twp, twh, tws, src, sliced, batch,
+                                                                   stream);
+    if (total >= kStreamXMinBatch)
+        return launch_fwd_passes<kColsWide, kRowsWide, true>(x, work, xs, twp, twh, tws, src, sliced, batch, stream);
     return launch_fwd_passes<kColsWide, kRowsWide>(x, work, xs, twp, twh, tws, src, sliced, batch, stream);
 }
 
-template <int CPW, int RPW, bool WT>
+template <int CPW, int RPW, Store SW, Store SY>
 static int launch_inv_passes(const float2* f, float2* work, float2* y, const float2* twp, const float2* twh,
                              const int* ovf, const float2* tws, int64_t batch, hipStream_t stream) {
-    hipLaunchKernelGGL((k_col_inv<CPW, WT>), dim3((unsigned)(batch * (256 / CPW))), dim3(8 * CPW), 0, stream, f,
+    hipLaunchKernelGGL((k_col_inv<CPW, SW>), dim3((unsigned)(batch * (256 / CPW))), dim3(8 * CPW), 0, stream, f,
                        work, twp, twh, ovf, tws);
     if (int e = launch_status()) return e;
-    hipLaunchKernelGGL((k_row_inv<RPW, WT>), dim3((unsigned)(batch * (128 / RPW))), dim3(16 * RPW), 0, stream, work,
+    hipLaunchKernelGGL((k_row_inv<RPW, SY>), dim3((unsigned)(batch * (128 / RPW))), dim3(16 * RPW), 0, stream, work,
                        y, tws);
     return launch_status();
 }
 
+// last: nothing reads y soon after (false: the sliced overlap-add does).
 static int inv_passes(const float2* f, float2* work, float2* y, const float2* twp, const float2* twh, const int* ovf,
-                      const float2* tws, int64_t batch, hipStream_t stream) {
+                      const float2* tws, int64_t batch, bool last, hipStream_t stream) {
+    constexpr Store P = Store::kPlain, T = Store::kThrough, N = Store::kStream;
     if (batch <= kNarrowMaxBatch)
-        return launch_inv_passes<kInvColsNarrow, kRowsNarrow, false>(f, work, y, twp, twh, ovf, tws, batch, stream);
+        return launch_inv_passes<kInvColsNarrow, kRowsNarrow, P, P>(f, work, y, twp, twh, ovf, tws, batch, stream);
     if (batch <= kInvWriteThroughMaxBatch)
-        return launch_inv_passes<kInvColsWide, kRowsWide, true>(f, work, y, twp, twh, ovf, tws, batch, stream);
-    return launch_inv_passes<kInvColsWide, kRowsWide, false>(f, work, y, twp, twh, ovf, tws, batch, stream);
+        return launch_inv_passes<kInvColsWide, kRowsWide, T, T>(f, work, y, twp, twh, ovf, tws, batch, stream);
+    if (last && batch >= kStreamYMinBatch)
+        return launch_inv_passes<kInvColsWide, kRowsWide, P, N>(f, work, y, twp, twh, ovf, tws, batch, stream);
+    return launch_inv_passes<kInvColsWide, kRowsWide, P, P>(f, work, y, twp, twh, ovf, tws, batch, stream);
 }
 
 // The inverse row pass with the sliced overlap-add in its store
@@ -138,13 +150,13 @@ __global__ __launch_bounds__(16 * RPW) void k_row_inv_ola(const float2* __restri
 static int col_inv_pass(const float2* f, float2* work, const float2* twp, const float2* twh, const int* ovf,
                         const float2* tws, int64_t batch, hipStream_t stream) {
     if (batch <= kNarrowMaxBatch)
-        hipLaunchKernelGGL((k_col_inv<kInvColsNarrow, false>), dim3((unsigned)(batch * (256 / kInvColsNarrow))),
+        hipLaunchKernelGGL((k_col_inv<kInvColsNarrow, Store::kPlain>), dim3((unsigned)(batch * (256 / kInvColsNarrow))),
                            dim3(8 * kInvColsNarrow), 0, stream, f, work, twp, twh, ovf, tws);
     else if (batch <= kInvWriteThroughMaxBatch)
-        hipLaunchKernelGGL((k_col_inv<kInvColsWide, true>), dim3((unsigned)(batch * (256 / kInvColsWide))),
+        hipLaunchKernelGGL((k_col_inv<kInvColsWide, Store::kThrough>), dim3((unsigned)(batch * (256 / kInvColsWide))),
                            dim3(8 * kInvColsWide), 0, stream, f, work, twp, twh, ovf, tws);
     else
-        hipLaunchKernelGGL((k_col_inv<kInvColsWide, false>), dim3((unsigned)(batch * (256 / kInvColsWide))),
+        hipLaunchKernelGGL((k_col_inv<kInvColsWide, Store::kPlain>), dim3((unsigned)(batch * (256 / kInvColsWide))),
                            dim3(8 * kInvColsWide), 0, stream, f, work, twp, twh, ovf, tws);
     return launch_status();
 }
@@ -207,11 +219,11 @@ extern "C" int fcqt_packed_fft_fwd(const fcqt_tables* tab, const float* x, float
     return fwd_passes(reinterpret_cast<const float2*>(x), reinterpret_cast<float2*>(work),
                       reinterpret_cast<float2*>(xs), reinterpret_cast<const float2*>(tab->tw_pass),
                       reinterpret_cast<const float2*>(tab->tw_half), reinterpret_cast<const float2*>(tab->tw_stage),
-                      SliceSrc{nullptr, nullptr, 1, 1, 0, 0, 0, nullptr, 1, 1, 1}, false, batch, stream);
+                      SliceSrc{nullptr, nullptr, 1, 1, 0, 0, 0, nullptr, 1, 1, 1}, false, batch, batch, stream);
 }
 
-extern "C" int fcqt_packed_fft_inv(const fcqt_tables* tab, const int32_t* ovf, const float* f, float* y,
-                                   float* work, int64_t batch, hipStream_t stream) {
+int fcqt::packed_fft_inv(const fcqt_tables* tab, const int32_t* ovf, const float* f, float* y, float* work,
+                         int64_t batch, bool last, hipStream_t stream) {
     if (!tab || !ovf || !f || !y || !work || batch < 1 || batch > kMaxBatch) return FCQT_EARG;
     if (!tab->tw_pass || !tab->tw_half || !tab->tw_stage) return FCQT_EARG;
     if (!aligned(f, 16) || !aligned(y, 8) || !aligned(work, 8) || !aligned(tab->tw_pass, 8) ||
@@ -220,12 +232,17 @@ extern "C" int fcqt_packed_fft_inv(const fcqt_tables* tab, const int32_t* ovf, c
     return inv_passes(reinterpret_cast<const float2*>(f), reinterpret_cast<float2*>(work),
                       reinterpret_cast<float2*>(y), reinterpret_cast<const float2*>(tab->tw_pass),
                       reinterpret_cast<const float2*>(tab->tw_half), reinterpret_cast<const int*>(ovf),
-                      reinterpret_cast<const float2*>(tab->tw_stage), batch, stream);
+                      reinterpret_cast<const float2*>(tab->tw_stage), batch, last, stream);
 }
 
-extern "C" int fcqt_slice_fft_fwd(const fcqt_tables* tab, const float* sig, int64_t sig_len, const float* window,
-                                  int64_t nsig, int64_t nslices, int64_t first, int64_t origin, float* xs,
-                                  float* work, hipStream_t stream) {
+extern "C" int fcqt_packed_fft_inv(const fcqt_tables* tab, const int32_t* ovf, const float* f, float* y,
+                                   float* work, int64_t batch, hipStream_t stream) {
+    return packed_fft_inv(tab, ovf, f, y, work, batch, false, stream);
+}
+
+int fcqt::slice_fft_fwd(const fcqt_tables* tab, const float* sig, int64_t sig_len, const float* window, int64_t nsig,
+                        int64_t nslices, int64_t first, int64_t origin, float* xs, float* work, int64_t total,
+                        hipStream_t stream) {
     if (!tab || !sig || !window || !xs || !work || sig_len < 1 || nsig < 1 || nslices < 1) return FCQT_EARG;
     if (first < 0 || first > kMaxBatch || origin < -(int64_t)kN || origin > (int64_t)kN * kMaxBatch)
         return FCQT_EARG;
@@ -242,7 +259,13 @@ extern "C" int fcqt_slice_fft_fwd(const fcqt_tables* tab, const float* sig, int6
                       reinterpret_cast<const float2*>(tab->tw_stage),
                       SliceSrc{sig, window, (long)sig_len, (int)nslices, (long)first, (long)origin, pairs, nullptr,
                                (long)sig_len, (long)sig_len, (long)sig_len},
-                      true, batch, stream);
+                      true, batch, total, stream);
+}
+
+extern "C" int fcqt_slice_fft_fwd(const fcqt_tables* tab, const float* sig, int64_t sig_len, const float* window,
+                                  int64_t nsig, int64_t nslices, int64_t first, int64_t origin, float* xs,
+                                  float* work, hipStream_t stream) {
+    return slice_fft_fwd(tab, sig, sig_len, window, nsig, nslices, first, origin, xs, work, nsig * nslices, stream);
 }
 
 extern "C" int fcqt_stream_analysis(const fcqt_tables* tab, const int32_t* route, const int32_t* groups,
@@ -271,7 +294,7 @@ extern "C" int fcqt_stream_analysis(const fcqt_tables* tab, const int32_t* route
                            reinterpret_cast<const float2*>(tab->tw_stage),
                            SliceSrc{prev, window, 2 * kHop, 1, (long)slice, kHop * ((long)slice - 1), pairs, next,
                                     (long)prev_stride, (long)next_stride, kHop},
-                           true, nsig, stream))
+                           true, nsig, nsig, stream))
         return e;
     return fcqt_route_bands_sliced(tab, route, groups, xs, coef, nsig, 1, slice, stream);
 }

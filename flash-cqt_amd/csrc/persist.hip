@@ -279,7 +279,7 @@ __global__ __launch_bounds__(kFlowThreads) __attribute__((amdgpu_waves_per_eu(4)
         } else if (stage == 2) {
             row_fwd_tile<kFRowsPerTile>((int)b, t, q.work, q.xs, q.twh, q.tws, lds, tid);
         } else {
-            route_task<LAYOUT, WT>(t, (int)b, q.xs, q.cre, q.cim, q.rec, q.tasks, q.ncoef, SliceMap{nullptr, 1, 0},
+            route_task<LAYOUT, WT ? Store::kThrough : Store::kPlain>(t, (int)b, q.xs, q.cre, q.cim, q.rec, q.tasks, q.ncoef, SliceMap{nullptr, 1, 0},
                                    q.tws, lds, tid);
         }
         trace_at(p, it, 3, clock100());
@@ -314,13 +314,13 @@ __global__ __launch_bounds__(kFlowThreads) void k_flow_synthesis(const FlowArgs 
         int tid;
         const FlowArgs q = flow_task_args(p, tid);
         if (stage == 1) {
-            scatter_task<LAYOUT, false>(t, (int)b, q.cre, q.cim, q.f, q.rec, q.tasks, q.ncoef,
+            scatter_task<LAYOUT>(t, (int)b, q.cre, q.cim, q.f, q.rec, q.tasks, q.ncoef,
                                         SliceMap{nullptr, 1, 0}, q.tws, lds, tid);
         } else if (stage == 2) {
-            col_inv_tile<kFInvColsPerTile, false>((int)b, t, reinterpret_cast<const float2*>(q.f), q.work, q.twp,
+            col_inv_tile<kFInvColsPerTile, Store::kPlain>((int)b, t, reinterpret_cast<const float2*>(q.f), q.work, q.twp,
                                                   q.twh, q.ovf, q.tws, lds, tid);
         } else {
-            row_inv_tile<kFRowsPerTile, WT>((int)b, t, q.work, q.y, q.tws, lds, tid);
+            row_inv_tile<kFRowsPerTile, WT ? Store::kThrough : Store::kPlain>((int)b, t, q.work, q.y, q.tws, lds, tid);
         }
         trace_at(p, it, 3, clock100());
         flow_done(p, stage, b);
