@@ -87,8 +87,7 @@ extern "C" int fcqt_stream_synthesis(const fcqt_tables* tab, const int32_t* scat
         !aligned(tail, 4) || (out && !aligned(out, 4)))
         return FCQT_EALIGN;
     if (int e = fcqt_scatter_bands_sliced(tab, scat, groups, coef, f, nsig, 1, slice, stream)) return e;
-    if (int e = fcqt_packed_fft_inv(tab, ovf, f, y, work, nsig, stream)) return e;
-    return fcqt_stream_overlap(y, tail, out, nsig, slice, stream);
+    return stream_inv_passes(tab, ovf, f, work, tail, out, nsig, slice, stream);
 }
 
 // ---------------------------------------------------------------------------

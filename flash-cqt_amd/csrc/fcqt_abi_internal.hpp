@@ -69,6 +69,12 @@ int slice_fft_fwd(const fcqt_tables* tab, const float* sig, int64_t sig_len, con
                   int64_t nslices, int64_t first, int64_t origin, float* xs, float* work, int64_t total,
                   hipStream_t stream);
 
+// The inverse passes of one streamed slice per signal with the half-slice
+// overlap-add in the row pass's store (arguments checked by the caller);
+// defined in packed_fft.hip.
+int stream_inv_passes(const fcqt_tables* tab, const int32_t* ovf, const float* f, float* work, float* tail, float* out,
+                      int64_t nsig, int64_t slice, hipStream_t stream);
+
 // Text of the last failed launch on this host thread.
 inline char* last_error_buf() {
     static thread_local char buf[256] = {0};

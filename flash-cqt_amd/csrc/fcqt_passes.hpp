@@ -443,19 +443,27 @@ __device__ __forceinline__ void row_inv_tile(const int b, const int rg, const fl
     }
 }
 
-// The inverse row pass of one slice s of a SlicedCQT signal with the
-// overlap-add in its store (whole-signal synthesis; orow is the signal's
-// output row of `length` samples). Slice s's samples jj, jj + 1 (jj =
-// 2 (kk1 + 128 k2)) go to p, p + 1 with p = 2H (s - 1) + j, j = (jj + H)
-// mod N in even slices and (jj - H) mod N in odd ones, where p < length.
-// Even slices (one launch) store 0 + v; odd slices (the next launch) add v
-// to that, or store 0 + v in their second half when there is no slice
-// s + 1. The values are the rounded products k_row_inv stores, so the sums
-// are k_overlap_add's (0 + a) + b up to the order of two operands, which
-// gives the same bits. PAIR: length even and orow 8-byte aligned, so p and
-// p + 1 are both in range or both out, and one 8-byte access serves both.
-template <int RPW, bool ODD, bool PAIR>
-__device__ __forceinline__ void row_inv_ola_tile(const int b, const int rg, const int s, const int S,
+// The inverse row pass over consecutive slices of a SlicedCQT signal with the
+// overlap-add in its store: one row tile (rows rg RPW ..) of the hops h0 ..
+// h1 - 1 of a signal of S slices, hop h being the output samples [2H h,
+// 2H (h + 1)) below `length`, the sum of slice h's second half and slice
+// h + 1's first half (slice S - 1's second half alone in the last hop). in and
+// orow are the signal's first work row and output row.
+//
+// A thread's 16 sample pairs of a slice lie at j = lane + 4096 u, lane = 2 (kk1 +
+// 128 kg) < 4096, and the quarter roll moves whole runs of 4096: pair u goes to
+// run (u + 4) mod 16 of the slice in even slices and (u + 12) mod 16 in odd
+// ones. So run i of a hop is u = i + 4 (mod 16, kHigh) or u = i + 12 (kLow) of
+// the same thread in every slice: it keeps a slice's second half in registers,
+// adds the next slice's first half and stores each output sample once, and no
+// slice ever goes to memory. Slice h1 is transformed again by the next tile of
+// the signal (its second half), so a tile of k hops costs k + 1 slices; the next
+// slice's rows are loaded while this one is transformed. The sums are
+// k_overlap_add's: (0 + a) + b of the rounded products k_row_inv stores.
+// PAIR: the rows of the output are 8-byte aligned, so a pair is one 8-byte
+// store (its second sample alone may lie past the end).
+template <int RPW, bool PAIR>
+__device__ __forceinline__ void row_inv_ola_tile(const int rg, const int h0, const int h1, const int S,
                                                  const long length, const float2* __restrict__ in,
                                                  float* __restrict__ orow, const float2* __restrict__ tws,
                                                  float2* lds, const int tid = threadIdx.x) {
@@ -463,33 +471,101 @@ __device__ __forceinline__ void row_inv_ola_tile(const int b, const int rg, cons
     float2* tw2 = lds + RPW * P::US;
     const int rho = tid >> 4;
     const int t = tid & 15;
-    row_fft_to_lds<false, false>(in + (long)b * kL + (long)(rg * RPW + rho) * 256, lds, tw2, rho, t, 16 * RPW, tws,
-                          nullptr, nullptr, tid);
-    const int rho2 = tid & (RPW - 1);
+    const float2* row = in + (rg * RPW + rho) * 256 + t;
+    float2* su = lds + rho * P::US;
     const int kg = tid / RPW;
-    const float2* s2 = lds + rho2 * P::US;
-    const int kk1 = rg * RPW + rho2;
+    const float2* s2 = lds + (tid & (RPW - 1)) * P::US + pad16(kg);   // pad16(kg + 16 u) = pad16(kg) + 17 u
+    const int lane = 2 * (rg * RPW + (tid & (RPW - 1)) + 128 * kg);
     constexpr float sc = 0.5f / (float)kL;     // 1/L of the inverse, 1/2 of the retangle
-    const long base = 2l * kQuarter * (s - 1);
-    const bool last = s + 1 >= S;              // no slice s + 1
+    load_tw2_lds<256>(tw2, tws, tid, 16 * RPW);
+    const int last = min(h1, S - 1);           // the last slice this tile needs
+    float2 v[16], next[16], carry[8];
 #pragma unroll
-    for (int u = 0; u < 16; ++u) {
-        const int k2 = kg + 16 * u;
-        const float2 w = s2[pad16(k2)];
-        const int j = (2 * (kk1 + 128 * k2) + (ODD ? kN - kQuarter : kQuarter)) & (kN - 1);
-        const long p = base + j;
-        float v0 = w.x * sc, v1 = -w.y * sc;
-        asm volatile("" : "+v"(v0), "+v"(v1));    // the rounded products, as k_row_inv stores them
-        const bool add = ODD && (j < 2 * kQuarter || !last);
-        if constexpr (PAIR) {
-            if (p >= 0 && p < length) {
-                float2* o = reinterpret_cast<float2*>(orow + p);
-                const float2 a = add ? *o : make_float2(0.0f, 0.0f);
-                *o = make_float2(a.x + v0, a.y + v1);
+    for (int r = 0; r < 16; ++r) next[r] = row[(long)h0 * kL + 16 * r];
+    for (int s = h0;; ++s) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) v[r] = next[r];
+        const long ahead = (long)min(s + 1, last) * kL;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) next[r] = row[ahead + 16 * r];
+        fft_unit<256, -1>(v, su, t, tw2, Tw3<256>{});
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 16; ++r) su[pad16(t + 16 * r)] = v[r];
+        __syncthreads();
+        const bool odd = s & 1;
+        const int first = odd ? 4 : 12, second = odd ? 12 : 4;     // u of run 0 of each half
+        float* o = orow + (2l * kQuarter * (s - 1) + lane);
+        const long room = length - (2l * kQuarter * (s - 1) + lane);    // samples from o to the end of the row
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float2 a = s2[17 * ((first + i) & 15)], b = s2[17 * ((second + i) & 15)];
+            float v0 = a.x * sc, v1 = -a.y * sc, w0 = b.x * sc, w1 = -b.y * sc;
+            asm volatile("" : "+v"(v0), "+v"(v1), "+v"(w0), "+v"(w1));    // the rounded products
+            if (s > h0) {
+                const float2 z = make_float2(carry[i].x + v0, carry[i].y + v1);
+                if (PAIR && room >= 4096 * i + 2) *reinterpret_cast<float2*>(o + 4096 * i) = z;
+                else {
+                    if (room > 4096 * i) o[4096 * i] = z.x;
+                    if (room > 4096 * i + 1) o[4096 * i + 1] = z.y;
+                }
             }
+            carry[i] = make_float2(0.0f + w0, 0.0f + w1);
+        }
+        if (s == last) break;
+        __syncthreads();                       // every pair read before the next slice overwrites the rows
+    }
+    if (h1 == S) {                             // the signal's last hop has no second slice
+        const long p = 2l * kQuarter * last + lane;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            if (p + 4096 * i < length) orow[p + 4096 * i] = carry[i].x;
+            if (p + 4096 * i + 1 < length) orow[p + 4096 * i + 1] = carry[i].y;
+        }
+    }
+}
+
+// The inverse row pass of one streamed slice with the half-slice overlap-add in
+// its store (k_stream_overlap's sums: out[p] = tail[p] + first half, tail[p] =
+// second half, emit = false: tail only). A thread holds both halves of the same
+// positions p (row_inv_ola_tile's runs), so it alone reads and replaces them.
+// PAIR: tail and out are 8-byte aligned.
+template <int RPW, bool PAIR>
+__device__ __forceinline__ void row_inv_stream_tile(const int rg, const bool odd, const bool emit,
+                                                    const float2* __restrict__ in, float* __restrict__ tail,
+                                                    float* __restrict__ out, const float2* __restrict__ tws,
+                                                    float2* lds, const int tid = threadIdx.x) {
+    using P = Plan<256>;
+    const int kg = tid / RPW;
+    const int lane = 2 * (rg * RPW + (tid & (RPW - 1)) + 128 * kg);
+    // the carried half, in flight with the row
+    float2 old[8];
+    if (emit) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            if constexpr (PAIR) old[i] = *reinterpret_cast<const float2*>(tail + lane + 4096 * i);
+            else old[i] = make_float2(tail[lane + 4096 * i], tail[lane + 4096 * i + 1]);
+        }
+    }
+    row_fft_to_lds<false, false>(in + (rg * RPW + (tid >> 4)) * 256, lds, lds + RPW * P::US, tid >> 4, tid & 15,
+                                 16 * RPW, tws, nullptr, nullptr, tid);
+    const float2* s2 = lds + (tid & (RPW - 1)) * P::US + pad16(kg);   // pad16(kg + 16 u) = pad16(kg) + 17 u
+    constexpr float sc = 0.5f / (float)kL;     // 1/L of the inverse, 1/2 of the retangle
+    const int first = odd ? 4 : 12, second = odd ? 12 : 4;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const float2 a = s2[17 * ((first + i) & 15)], b = s2[17 * ((second + i) & 15)];
+        float v0 = a.x * sc, v1 = -a.y * sc;
+        asm volatile("" : "+v"(v0), "+v"(v1));    // the rounded products, as k_row_inv stores them
+        const float2 z = make_float2(old[i].x + v0, old[i].y + v1), w = make_float2(b.x * sc, -b.y * sc);
+        float* tp = tail + lane + 4096 * i;
+        float* op = out + lane + 4096 * i;
+        if constexpr (PAIR) {
+            if (emit) *reinterpret_cast<float2*>(op) = z;
+            *reinterpret_cast<float2*>(tp) = w;
         } else {
-            if (p >= 0 && p < length) orow[p] = (add ? orow[p] : 0.0f) + v0;
-            if (p + 1 >= 0 && p + 1 < length) orow[p + 1] = (add ? orow[p + 1] : 0.0f) + v1;
+            if (emit) op[0] = z.x, op[1] = z.y;
+            tp[0] = w.x, tp[1] = w.y;
         }
     }
 }

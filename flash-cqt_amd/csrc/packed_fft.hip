@@ -129,21 +129,37 @@ static int inv_passes(const float2* f, float2* work, float2* y, const float2* tw
     return launch_inv_passes<kInvColsWide, kRowsWide, P, P>(f, work, y, twp, twh, ovf, tws, batch, stream);
 }
 
-// The inverse row pass with the sliced overlap-add in its store
-// (row_inv_ola_tile): the slices of one parity of nsig signals x S slices,
-// nper of them per signal; work row sig * S + s, output row sig of `length`.
-template <int RPW, bool ODD, bool PAIR>
+// The inverse row pass of a whole sliced signal with the overlap-add in its
+// store (row_inv_ola_tile): tiles of `hops` hops of the `nhops` that the output
+// of `length` samples has.
+template <int RPW, bool PAIR>
 __global__ __launch_bounds__(16 * RPW) void k_row_inv_ola(const float2* __restrict__ in, float* __restrict__ out,
                                                           const float2* __restrict__ tws, int S, long length,
-                                                          int nper) {
+                                                          int nhops, int hops) {
+    constexpr int kWgs = 128 / RPW;               // row tiles
+    __shared__ float2 lds[row_lds<RPW>()];
+    const int lg = xcd_remap((int)blockIdx.x, (int)gridDim.x);
+    const int per = (nhops + hops - 1) / hops;    // hop tiles per signal
+    const int r = lg / kWgs;                      // sig * per + hop tile
+    const int sig = r / per;
+    const int h0 = (r - sig * per) * hops;
+    row_inv_ola_tile<RPW, PAIR>(lg - r * kWgs, h0, min(h0 + hops, nhops), S, length, in + (long)sig * S * kL,
+                                out + (long)sig * length, tws, lds);
+}
+
+// The inverse row pass of one streamed slice per signal (row_inv_stream_tile).
+// At 8 signals it took the row pass and k_stream_overlap 4.0 + 2.6 us and a
+// launch between them.
+template <int RPW, bool PAIR>
+__global__ __launch_bounds__(16 * RPW) void k_row_inv_stream(const float2* __restrict__ in, float* __restrict__ tail,
+                                                             float* __restrict__ out,
+                                                             const float2* __restrict__ tws, int odd, int emit) {
     constexpr int kWgs = 128 / RPW;               // workgroups per slice
     __shared__ float2 lds[row_lds<RPW>()];
     const int lg = xcd_remap((int)blockIdx.x, (int)gridDim.x);
-    const int r = lg / kWgs;                      // sig * nper + m: slice s = 2 m + ODD of signal sig
-    const int sig = r / nper;
-    const int s = 2 * (r - sig * nper) + (ODD ? 1 : 0);
-    row_inv_ola_tile<RPW, ODD, PAIR>(sig * S + s, lg - r * kWgs, s, S, length, in, out + (long)sig * length, tws,
-                                     lds);
+    const int b = lg / kWgs;
+    row_inv_stream_tile<RPW, PAIR>(lg - b * kWgs, odd, emit, in + (long)b * kL, tail + (long)b * 2 * kQuarter,
+                                   out + (long)b * 2 * kQuarter, tws, lds);
 }
 
 // The inverse column pass alone, in the shape inv_passes picks for the batch.
@@ -161,19 +177,51 @@ static int col_inv_pass(const float2* f, float2* work, const float2* twp, const 
     return launch_status();
 }
 
-// Both parities of the fused row pass: the even slices' launch, then the odd.
+// Hops per tile for a call of `total` hops: as few as fill the chip, since a tile
+// of k hops transforms k + 1 slices; longer tiles once there are more tiles than
+// the chip holds at once. SlicedCQT.bwd with 1 / 2 / 3 / 4 / 6 hops per tile (us):
+// 15 hops 23.1 / 24.7 / 27.1 / 29.3 / 34.3, 112 75.6 / 76.2 / 76.5 / 78.4 / 83.4,
+// 156 96.4 / 95.9 / 95.9 / 98.2 / 100.4, 223 128.7 / 127.5 / 127.7 / 126.9 / 132.3,
+// 511 308.3 / 307.4 / 306.4 / 302.7 / 302.9. The row pass into a slice buffer and
+// an overlap-add kernel took 31.5, 79.3, 101.1 and 142.2 us, the even and odd
+// slices in two read-add-store launches 313.3 us at 511 hops.
+static int64_t ola_hops(int64_t total) { return total < 160 ? 1 : (total < 320 ? 2 : 4); }
+
 template <int RPW, bool PAIR>
-static int row_inv_ola_passes(const float2* work, float* out, const float2* tws, int64_t nsig, int64_t S,
-                              int64_t length, hipStream_t stream) {
-    constexpr int kWgs = 128 / RPW;
-    const int64_t even = (S + 1) / 2, odd = S / 2;
-    hipLaunchKernelGGL((k_row_inv_ola<RPW, false, PAIR>), dim3((unsigned)(nsig * even * kWgs)), dim3(16 * RPW), 0,
-                       stream, work, out, tws, (int)S, (long)length, (int)even);
-    if (int e = launch_status()) return e;
-    if (odd == 0) return FCQT_OK;
-    hipLaunchKernelGGL((k_row_inv_ola<RPW, true, PAIR>), dim3((unsigned)(nsig * odd * kWgs)), dim3(16 * RPW), 0,
-                       stream, work, out, tws, (int)S, (long)length, (int)odd);
+static int row_inv_ola_pass(const float2* work, float* out, const float2* tws, int64_t nsig, int64_t S, int64_t length,
+                            hipStream_t stream) {
+    constexpr int64_t kWgs = 128 / RPW, kHop = 2 * kQuarter;
+    const int64_t nhops = (length + kHop - 1) / kHop;
+    const int64_t hops = ola_hops(nsig * nhops);
+    const int64_t grid = nsig * ((nhops + hops - 1) / hops) * kWgs;
+    hipLaunchKernelGGL((k_row_inv_ola<RPW, PAIR>), dim3((unsigned)grid), dim3(16 * RPW), 0, stream, work, out, tws,
+                       (int)S, (long)length, (int)nhops, (int)hops);
     return launch_status();
+}
+
+template <int RPW, bool PAIR>
+static int row_inv_stream_pass(const float2* work, float* tail, float* out, const float2* tws, int64_t nsig,
+                               int64_t slice, hipStream_t stream) {
+    hipLaunchKernelGGL((k_row_inv_stream<RPW, PAIR>), dim3((unsigned)(nsig * (128 / RPW))), dim3(16 * RPW), 0, stream,
+                       work, tail, out, tws, (int)(slice & 1), slice > 0 ? 1 : 0);
+    return launch_status();
+}
+
+int stream_inv_passes(const fcqt_tables* tab, const int32_t* ovf, const float* f, float* work, float* tail, float* out,
+                      int64_t nsig, int64_t slice, hipStream_t stream) {
+    const auto* tws = reinterpret_cast<const float2*>(tab->tw_stage);
+    auto* w2 = reinterpret_cast<float2*>(work);
+    if (int e = col_inv_pass(reinterpret_cast<const float2*>(f), w2, reinterpret_cast<const float2*>(tab->tw_pass),
+                             reinterpret_cast<const float2*>(tab->tw_half), reinterpret_cast<const int*>(ovf), tws,
+                             nsig, stream))
+        return e;
+    if (!out) out = tail;                         // slice 0 stores no output
+    const bool pair = aligned(tail, 8) && aligned(out, 8);
+    if (nsig <= kNarrowMaxBatch)
+        return pair ? row_inv_stream_pass<kRowsNarrow, true>(w2, tail, out, tws, nsig, slice, stream)
+                    : row_inv_stream_pass<kRowsNarrow, false>(w2, tail, out, tws, nsig, slice, stream);
+    return pair ? row_inv_stream_pass<kRowsWide, true>(w2, tail, out, tws, nsig, slice, stream)
+                : row_inv_stream_pass<kRowsWide, false>(w2, tail, out, tws, nsig, slice, stream);
 }
 
 }  // namespace fcqt
@@ -201,12 +249,12 @@ extern "C" int fcqt_sliced_synthesis(const fcqt_tables* tab, const int32_t* scat
                              reinterpret_cast<const float2*>(tab->tw_half), reinterpret_cast<const int*>(ovf), tws,
                              batch, stream))
         return e;
-    const bool pair = length % 2 == 0 && aligned(out, 8);
+    const bool pair = (length % 2 == 0 || nsig == 1) && aligned(out, 8);
     if (batch <= kNarrowMaxBatch)
-        return pair ? row_inv_ola_passes<kRowsNarrow, true>(w2, out, tws, nsig, nslices, length, stream)
-                    : row_inv_ola_passes<kRowsNarrow, false>(w2, out, tws, nsig, nslices, length, stream);
-    return pair ? row_inv_ola_passes<kRowsWide, true>(w2, out, tws, nsig, nslices, length, stream)
-                : row_inv_ola_passes<kRowsWide, false>(w2, out, tws, nsig, nslices, length, stream);
+        return pair ? row_inv_ola_pass<kRowsNarrow, true>(w2, out, tws, nsig, nslices, length, stream)
+                    : row_inv_ola_pass<kRowsNarrow, false>(w2, out, tws, nsig, nslices, length, stream);
+    return pair ? row_inv_ola_pass<kRowsWide, true>(w2, out, tws, nsig, nslices, length, stream)
+                : row_inv_ola_pass<kRowsWide, false>(w2, out, tws, nsig, nslices, length, stream);
 }
 
 extern "C" int fcqt_packed_fft_fwd(const fcqt_tables* tab, const float* x, float* xs, float* work,

@@ -16,9 +16,8 @@ pure-torch one. Assigning self.cqt swaps engines as in the reference.
 With the HIP engine and no gradient to record, fwd and bwd run the framing
 inside the engine's kernels (fcqt_sliced_analysis, which frames, transforms
 and routes, in chunks of about 128 slices from 256 slices on;
-fcqt_scatter_bands_sliced, the inverse passes and fcqt_overlap_add, or from
-256 slices on fcqt_sliced_synthesis, which overlap-adds in the inverse row
-pass's store): slices are read straight from the signal, coefficients are
+fcqt_sliced_synthesis, which overlap-adds in the inverse row pass's store):
+slices are read straight from the signal, coefficients are
 written and read in the block layout with the quarter roll applied, and the
 inverse slices are rolled and overlap-added in one pass. Blocks returned by that path are views of one buffer; passing
 them back to bwd reads that buffer without a copy. The bounded-state stream
@@ -39,13 +38,11 @@ from .oct_cqt import OctCQT
 
 # From this many slices on the whole-signal synthesis overlap-adds in the
 # inverse row pass (fcqt_sliced_synthesis); below, the slices go through a
-# slice buffer and one overlap-add kernel, which measured faster there
-# (SlicedCQT.bwd, fused against buffered): 53 against 49 us at 64 slices;
-# at configs[4]'s 120 slices the two row-pass launches took 8.4 + 12.7 us
-# against 11.3 + 8.2 us for the row pass and the overlap-add; 170 against
-# 179 us at 256 slices and 327-336 against 353-364 us at 512. Same bits
-# either way.
-FUSED_OLA_MIN_SLICES = 256
+# slice buffer and one overlap-add kernel. The row pass measured faster at
+# every size (SlicedCQT.bwd, fused against buffered): 23 against 32 us up to 15
+# slices, 75.6 against 79.3 us at 120 and 127 against 142 us at 224. Same
+# bits either way.
+FUSED_OLA_MIN_SLICES = 1
 
 
 def makewnd(sl_len, tr_area, device="cpu", dtype=torch.float32):

@@ -384,8 +384,8 @@ int fcqt_scatter_bands_sliced(const fcqt_tables* tab, const int32_t* scat, const
 
 /* The whole-signal sliced synthesis in one call, with the overlap-add in the
  * inverse row pass: fcqt_scatter_bands_sliced (first = 0), the inverse column
- * pass, then the inverse row pass twice, over the even slices (storing into
- * out) and over the odd ones (adding to it), so no [nslices][65536] slice
+ * pass, then an inverse row pass whose workgroups walk consecutive slices of a
+ * signal and carry each slice's second half, so no [nslices][65536] slice
  * buffer is written or read back. The same output bits as
  * fcqt_scatter_bands_sliced + fcqt_packed_fft_inv + fcqt_overlap_add.
  *   coef   nsig * nslices * ncoef complex, the block layout
@@ -437,9 +437,10 @@ int fcqt_stream_analysis(const fcqt_tables* tab, const int32_t* route, const int
                          float* work, hipStream_t stream);
 
 /* One streamed synthesis step: fcqt_scatter_bands_sliced (one slice per
- * signal, first = slice), fcqt_packed_fft_inv and fcqt_stream_overlap in one
- * call, with every argument checked before the first launch. out may be NULL
- * for slice 0.
+ * signal, first = slice), the inverse passes and the sums of
+ * fcqt_stream_overlap in the row pass's store (y, a slice buffer as that call
+ * takes, is required but not used), with every argument checked before the
+ * first launch. out may be NULL for slice 0.
  * Replaces the per-slice step of SlicedCQT.stream_bwd (sliced.py:194-209):
  * _arrange, inv_bands, inv_tail, the roll and the half-slice overlap-add. */
 int fcqt_stream_synthesis(const fcqt_tables* tab, const int32_t* scat, const int32_t* groups,
