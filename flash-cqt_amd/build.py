@@ -6,7 +6,9 @@ Output: flash-cqt_amd/flash_cqt/_lib/libflashcqt.so, and beside it two
 variant libraries of the same sources: libflashcqt_xlane.so (the band units of
 M <= 256 exchanging across lanes instead of through LDS; the benchmark and the
 GPU tests compare the two) and libflashcqt_flowtrace.so (the single-launch
-kernels stamping a stage trace, fcqt_persist_trace). All compile in parallel. Flags: -O3 for gfx950,
+kernels stamping a stage trace, fcqt_persist_trace), and _fcqt_torch.so, the
+host glue of TrainableCQT and SlicedCQT (g++, no device code). All compile in
+parallel. Flags: -O3 for gfx950,
 packed fp32 instructions disabled (-Xclang -target-feature -Xclang
 -packed-fp32-ops). The host pass warns that it does not know the packed-fp32
 feature; that warning is harmless.
@@ -65,6 +67,24 @@ def resource_usage(text):
     return out
 
 
+GLUE_SOURCE = CSRC / "torch_glue.cpp"
+GLUE = OUT.with_name("_fcqt_torch.so")
+
+
+def glue_command(out=GLUE):
+    """The host glue: a Python extension module against torch's own headers
+    and libraries (no device code, so the host compiler)."""
+    import sysconfig
+    import torch
+    base = pathlib.Path(torch.__file__).resolve().parent
+    inc = [base / "include", base / "include" / "torch" / "csrc" / "api" / "include",
+           sysconfig.get_paths()["include"], "/opt/rocm/include"]
+    return [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__",
+            "-DUSE_ROCM", "-DTORCH_EXTENSION_NAME=_fcqt_torch", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+            *[a for d in inc for a in ("-isystem", str(d))], str(GLUE_SOURCE), "-o", str(out), f"-L{base / 'lib'}",
+            "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python", "-lc10", "-lc10_hip"]
+
+
 def build(verbose=False):
     """Compile the library and its variants (in parallel); returns the
     library's path. Fails on a compile error or on any kernel that uses
@@ -78,6 +98,8 @@ def build(verbose=False):
         procs[name] = (out, tmp, cmd, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT,
                                                        text=True))
     failed = []
+    glue_tmp = GLUE.with_suffix(".so.tmp")
+    glue = subprocess.Popen(glue_command(glue_tmp), stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     for name, (out, tmp, cmd, proc) in procs.items():
         text, _ = proc.communicate()
         lines = [ln for ln in text.splitlines()
@@ -101,6 +123,13 @@ def build(verbose=False):
                 for k, v in sorted(usage.items()):
                     f.write(k + " " + " ".join(f"{a}={b}" for a, b in v.items()) + "\n")
         os.replace(tmp, out)
+    text, _ = glue.communicate()
+    if verbose or glue.returncode != 0:
+        print(text)
+    if glue.returncode != 0:
+        failed.append(f"host glue: compiler failed ({glue.returncode})")
+    else:
+        os.replace(glue_tmp, GLUE)
     if failed:
         raise RuntimeError("; ".join(failed))
     return OUT

@@ -7,11 +7,13 @@ capture valid for its launches. There is no fallback: if the library is
 missing or does not load, every engine entry point raises.
 """
 import ctypes
+import importlib.util
 import pathlib
 
 import torch
 
 LIB_PATH = pathlib.Path(__file__).resolve().parent / "_lib" / "libflashcqt.so"
+GLUE_PATH = LIB_PATH.with_name("_fcqt_torch.so")
 ABI_VERSION = 13
 SYNC_PER_SLICE = 64       # FCQT_SYNC_PER_SLICE: uint32 per slice in a single-launch counter buffer
 SYNC_HEAD_WORDS = 320     # FCQT_SYNC_HEAD_WORDS: the error word, exit count and per-XCD queue claims
@@ -90,6 +92,21 @@ def load_variant(name):
             raise NativeError(f"unknown library variant {name!r}")
         _variants[name] = _open(LIB_PATH.with_name(VARIANTS[name]))
     return _variants[name]
+
+
+_glue = None
+
+
+def load_glue():
+    """The host glue module (csrc/torch_glue.cpp) that TrainableCQT and
+    SlicedCQT call where one C++ call replaces many small Python ones, or None
+    when it was not built: the Python paths then do the same work."""
+    global _glue
+    if _glue is None and GLUE_PATH.exists():
+        spec = importlib.util.spec_from_file_location("_fcqt_torch", GLUE_PATH)
+        _glue = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(_glue)
+    return _glue
 
 
 def _open(path):

@@ -18,6 +18,8 @@ No result is accumulated with atomics (every output value has one writer):
 every result is bitwise reproducible.
 Table semantics follow fused.py:303-476; see flash_cqt/tables.py.
 """
+import ctypes
+
 import numpy as np
 import torch
 
@@ -120,6 +122,7 @@ class FusedOctCQT:
         self._recorded = []    # sets a captured graph still uses
         self._ws = {}          # batch size -> views of the set's leading rows
         self._wp = {}          # batch size -> their raw pointers
+        self._glue = None      # the C++ host glue that uses the current set too
 
     # ------------------------------------------------------------ buffers
 
@@ -144,11 +147,8 @@ class FusedOctCQT:
         its addresses and use them on every replay."""
         full = self._full
         if full is None or full["B"] < B:
-            if full is not None and full["captured"]:
-                self._recorded.append(full)
-            self._ws.clear()
-            self._wp.clear()
-            self._full = full = None       # release the old set before allocating the new one
+            self._drop_set()               # release the old set before allocating the new one
+            full = None
             with torch.cuda.device(self.dev):
                 e = lambda *s: torch.empty(*s, dtype=torch.float32, device=self.dev)
                 z = lambda *s: torch.zeros(*s, dtype=torch.float32, device=self.dev)
@@ -164,6 +164,7 @@ class FusedOctCQT:
                 self._full = full = dict(B=B, captured=False, X=e(B, T.XSTRIDE, 2), W=e(B, L, 2),
                                          F=slot_buffer(B, self.dev), KR=planes[:n], KI=planes[n + SKEW:],
                                          XO=z(B, N))
+            self._publish()
         if B not in self._ws:
             nc = B * self.ncoef
             w = dict(X=full["X"][:B], W=full["W"][:B], F=full["F"][:B],
@@ -182,11 +183,39 @@ class FusedOctCQT:
     def release_workspace(self):
         """Drop the engine's buffer set (a set recorded by a graph capture
         stays with the graph's engine); the next call allocates afresh."""
-        if self._full is not None and self._full["captured"]:
-            self._recorded.append(self._full)
-        self._full = None
+        self._drop_set()
+
+    def _drop_set(self):
+        full = self._full
+        if full is not None and (full["captured"] or (self._glue is not None and self._glue.captured)):
+            self._recorded.append(full)
         self._ws.clear()
         self._wp.clear()
+        self._full = None
+        if self._glue is not None:
+            self._glue.clear_workspace()
+
+    def _publish(self):
+        """Tell the host glue about the current set (or a buffer added to it)."""
+        full = self._full
+        if self._glue is not None and full is not None:
+            self._glue.set_workspace(full["B"], full["X"], full["W"], full["F"], full.get("FA"))
+
+    def attach_glue(self):
+        """The host glue object of this engine (csrc/torch_glue.cpp), which runs
+        interleaved directions with this engine's tables and buffer set; None
+        when the glue is not built."""
+        mod = _native.load_glue()
+        if mod is None or self._glue is not None:
+            return self._glue
+        up, t = self._up, self._ct
+        fn = lambda f: ctypes.cast(f, ctypes.c_void_p).value
+        self._glue = mod.Engine([t.tw_pass, t.tw_half, t.tw_stage, t.tasks, up.route, up.route_b, up.scat, up.scat_a,
+                                 up.ovf_scat, up.ovf_scat_a], t.ntasks, t.ncoef, t.coef_span,
+                                fn(self.lib.fcqt_analysis), fn(self.lib.fcqt_synthesis), self._table_mem,
+                                [list(g) for g in self.gspec], len(self.cqt.groups))
+        self._publish()
+        return self._glue
 
     def _add_full(self, name, make):
         """Add a lazily allocated buffer (FA, SYNC) to the current set and to
@@ -198,6 +227,7 @@ class FusedOctCQT:
             for B, w in self._ws.items():
                 w[name] = full[name][:B] if name != "SYNC" else full[name][:_native.sync_words(B)]
                 self._wp[B][name] = w[name].data_ptr()
+            self._publish()
 
     def fa_buffer(self, B):
         """The analysis-adjoint scatter buffer for batch B, allocated and

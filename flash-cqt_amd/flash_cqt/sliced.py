@@ -289,14 +289,22 @@ class SlicedCQT:
         coef = torch.empty(nsig * S * f.ncoef, dtype=torch.complex64, device=f.dev)
         f.sliced_analysis(sig, self._tw32(), S, coef, ws["X"], ws["W"])
         ng = len(self.oct_bins)
-        blocks, side = [], []
+        args = []
         for gi, (b, M, off) in enumerate(f.gspec):
-            v = coef[nsig * S * off:nsig * S * (off + b * M)]
-            if gi < ng:
-                blocks.append(v.view(B, C, b, S * M))
-            else:
-                side.append(v.view(B, C, S, b, M))
-        return blocks, side
+            n = S * M
+            args.append(((B, C, b, n), (C * b * n, b * n, n, 1), nsig * S * off) if gi < ng else
+                        ((B, C, S, b, M), (C * b * n, b * n, b * M, M, 1), nsig * S * off))
+        views = self._views(coef, args)
+        return views[:ng], views[ng:]
+
+    @staticmethod
+    def _views(coef, args):
+        """as_strided views of one coefficient buffer, in one call where the
+        host glue is built."""
+        glue = _native.load_glue()
+        if glue is not None and not torch.compiler.is_compiling():
+            return glue.strided_views(coef, args)
+        return [coef.as_strided(*a) for a in args]
 
     def _block_buffer(self, f, blocks, side, nsig, S):
         """One complex64 buffer in the fused block layout: the blocks' own
@@ -422,7 +430,7 @@ class SlicedCQT:
         _native.check(f.lib.fcqt_stream_analysis(f._ct, f._tp["route"], f._tp["slice_groups"], pv.data_ptr(), ps,
                                                  cv.data_ptr(), cs, st["tw"], nsig, k, coef.data_ptr(), st["X"],
                                                  st["W"], _native.stream_handle(f.dev.index)), "stream_analysis")
-        views = self._stream_mark(f, [coef.as_strided(*a) for a in self._stream_view_args(f, B, C)])
+        views = self._stream_mark(f, self._views(coef, self._stream_view_args(f, B, C)))
         ng = len(self.oct_bins)
         return views[:ng], views[ng:]
 

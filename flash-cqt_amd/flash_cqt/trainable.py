@@ -31,13 +31,26 @@ class TrainableCQT:
         self.gspec = self.f.gspec
         self.ncoef = self.f.ncoef
         self.ngroups = len(cqt.groups)
+        self._lib = self.f.lib             # the library the glue's entry points belong to
+        self._glue = self.f.attach_glue()
+
+    def _plain(self, tensors):
+        """The host glue when every tensor is an ordinary one and the engine
+        runs the library it was attached to (the glue itself declines what
+        else it does not take), else None."""
+        if self._glue is not None and self.f.lib is self._lib and not torch.compiler.is_compiling() \
+                and all(type(t) is torch.Tensor or type(t) is torch.nn.Parameter for t in tensors):
+            return self._glue
+        return None
 
     # ------------------------------------------------ engine directions
     # The inputs reaching these are [B, N] float32 or [B, ncoef] complex64,
     # contiguous and on the engine's device (fwd/bwd and the autograd
     # Functions make them so); outputs are fresh buffers of the right size.
     # So the launches go straight to the C ABI with the engine's cached
-    # workspace and table pointers.
+    # workspace and table pointers. fwd and bwd hand ordinary calls to the
+    # host glue (csrc/torch_glue.cpp: the same launches, views and gradients
+    # from one C++ call); these methods serve the calls it declines.
 
     def _launch_analysis(self, x, table):
         B = x.shape[0]
@@ -77,6 +90,10 @@ class TrainableCQT:
 
     def fwd(self, x):
         """x [..., N] real -> (blocks, side) complex views, gradients flow."""
+        glue = self._plain((x,))
+        out = glue.fwd(x) if glue is not None else None
+        if out is not None:
+            return out
         lead = x.shape[:-1]
         xf = x.reshape(-1, N)
         if xf.dtype != torch.float32:
@@ -107,6 +124,12 @@ class TrainableCQT:
 
     def bwd(self, blocks, side=None):
         """Inverse of fwd; side=None treats the DC and Nyquist bands as zero."""
+        if side is not None:
+            parts = list(blocks) + list(side)
+            glue = self._plain(parts)
+            out = glue.bwd(parts) if glue is not None else None
+            if out is not None:
+                return out
         lead = blocks[0].shape[:-2]
         B = 1
         for d in lead:

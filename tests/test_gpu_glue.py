@@ -1,0 +1,117 @@
+"""TrainableCQT through the host glue against its Python path: the same bits and
+gradients for the calls that the glue takes, and the same answers, errors
+included, for those it declines."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+N = 65536
+
+
+@pytest.fixture(scope="module")
+def pair():
+    """(glue, Python path): two engines of one layout."""
+    from flash_cqt import OctCQT
+    from flash_cqt.trainable import TrainableCQT
+    cqt = OctCQT([3, 4, 2], [8, 16, 32], fs=44100, audio_len=N, device="cuda:0")
+    a, b = TrainableCQT(cqt, "cuda:0"), TrainableCQT(cqt, "cuda:0")
+    assert a._glue is not None, "the host glue is built by __graft_entry__.build()"
+    b._glue = None
+    return a, b
+
+
+def _x(*lead, seed=0, dtype=torch.float32):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    return torch.randn(*lead, N, generator=g, device="cuda").to(dtype)
+
+
+def _same(p, q):
+    return len(p) == len(q) and all(a.shape == b.shape and a.dtype == b.dtype and torch.equal(a, b)
+                                    for a, b in zip(p, q))
+
+
+def _step(t, x, edit):
+    x = x.detach().requires_grad_(True)
+    blocks, side = t.fwd(x)
+    if edit == "in place":
+        blocks[3].mul_(0.5)
+    elif edit == "new":
+        blocks = [c * (i + 1.0) for i, c in enumerate(blocks)]
+    elif edit == "swap":                       # views of the right buffer in another order of slices
+        blocks, side = [c.transpose(0, 1) for c in blocks], [c.transpose(0, 1) for c in side]
+        blocks, side = [c.contiguous() for c in blocks], [c.contiguous() for c in side]
+    y = t.bwd(blocks, None if edit == "no side" else side)
+    loss = (y * y).sum() + blocks[0].abs().sum() + blocks[2].conj().real.sum()
+    g, = torch.autograd.grad(loss, x)
+    return [*[c.detach() for c in blocks], *[c.detach() for c in side], y.detach(), g]
+
+
+@pytest.mark.parametrize("edit", ["none", "in place", "new", "no side"])
+@pytest.mark.parametrize("lead,dtype", [((1,), torch.float32), ((5,), torch.float32), ((2, 3), torch.float32),
+                                        ((), torch.float32), ((2, 1), torch.float64)])
+def test_glue_step_equals_python_path(pair, lead, dtype, edit):
+    x = _x(*lead, seed=len(lead), dtype=dtype)
+    assert _same(_step(pair[0], x, edit), _step(pair[1], x, edit))
+    assert _same(_step(pair[0], x, edit), _step(pair[1], x, edit))     # with every buffer of the set there
+
+
+def test_glue_takes_slices_in_the_order_given(pair):
+    assert _same(_step(pair[0], _x(2, 3), "swap"), _step(pair[1], _x(2, 3), "swap"))
+    blocks, side = pair[0].fwd(_x(2, 3))
+    turned = pair[0].bwd([c.transpose(0, 1) for c in blocks], [c.transpose(0, 1) for c in side])
+    assert torch.equal(turned, pair[0].bwd(blocks, side).transpose(0, 1))
+
+
+def test_glue_no_grad_strided_and_conjugated_inputs(pair):
+    for x in (_x(4)[1:3], _x(4)[::2], _x(3).conj().real, -_x(2), torch.complex(_x(2), _x(2, seed=1)).conj().imag):
+        with torch.no_grad():
+            (b, s), (b2, s2) = pair[0].fwd(x), pair[1].fwd(x)
+            assert _same([*b, *s], [*b2, *s2])
+            assert torch.equal(pair[0].bwd(b, s), pair[1].bwd(b2, s2))
+
+
+def test_glue_backward_after_the_engine_and_its_buffers_are_gone():
+    from flash_cqt import OctCQT
+    from flash_cqt.trainable import TrainableCQT
+    cqt = OctCQT([3, 4, 2], [8, 16, 32], fs=44100, audio_len=N, device="cuda:0")
+    t = TrainableCQT(cqt, "cuda:0")
+    ref = _step(t, _x(3), "none")[-1]
+    x = _x(3).requires_grad_(True)
+    blocks, side = t.fwd(x)
+    loss = (t.bwd(blocks, side) ** 2).sum() + blocks[0].abs().sum() + blocks[2].conj().real.sum()
+    t.fwd(_x(6))                               # a larger set replaces the one of the forward pass
+    t.f.release_workspace()
+    del t
+    junk = [torch.full((1 << 22,), float("nan"), device="cuda") for _ in range(16)]
+    assert torch.equal(torch.autograd.grad(loss, x)[0], ref)
+    del junk
+
+
+def test_glue_declines_what_the_python_path_refuses(pair):
+    for t in pair:
+        with pytest.raises(ValueError):
+            t.fwd(torch.randn(2, N))
+        with pytest.raises(ValueError):
+            t.fwd(torch.empty(0, N, device="cuda"))
+        b, s = t.fwd(_x(2))
+        with pytest.raises(ValueError):
+            t.bwd([c[..., :-1] for c in b], s)
+        with pytest.raises(RuntimeError):      # no forward-mode rule
+            torch.func.jvp(lambda v: t.fwd(v)[0][0], (_x(1),), (_x(1),))
+        with pytest.raises(RuntimeError):      # no batching rule
+            torch.func.vmap(lambda v: t.fwd(v)[0][0])(_x(2, 1))
+
+
+def test_glue_step_in_a_graph_and_from_threads(pair):
+    from concurrent.futures import ThreadPoolExecutor
+    from flash_cqt import Graphed
+    t = pair[0]
+    x = _x(4)
+    want = t.bwd(*t.fwd(x))
+    g = Graphed(lambda a: t.bwd(*t.fwd(a)), x)
+    t.fwd(_x(9))                               # the recorded set stays with the graph
+    for _ in range(3):
+        assert torch.equal(g(x), want)
+    torch.cuda.synchronize()
+    with ThreadPoolExecutor(4) as pool:        # on one stream
+        assert all(torch.equal(y, want) for y in pool.map(lambda i: t.bwd(*t.fwd(x)), range(16)))
