@@ -32,8 +32,8 @@ Everything the kernels need that does not depend on the batch:
            ranked; ranks 0 and 1 own the bin's slot in dense plane 0 or 1
            (F[r FSTRIDE + bin]: the taps of one band and rank are contiguous,
            so a band writes whole cache lines), ranks 2-3 own two slots of a
-           compact overflow area indexed by the bin's position among the bins
-           of degree > 2. Every slot has one writer, the set of written slots
+           compact overflow area indexed by the bin's place in the fold
+           lists. Every slot has one writer, the set of written slots
            is fixed by the table, and slots never written stay zero, so F
            needs zeroing only once.
   ovf_*    per scatter table, int32 [8][512] fold lists for the inverse
@@ -276,7 +276,7 @@ def scatter_table(bins, gr, gi):
     obins = np.flatnonzero(deg > 2)
     assert obins.size <= OVF_CAP, "overflow area too small"
     oidx = np.full(L + 1, -1, dtype=np.int64)
-    oidx[obins] = np.arange(obins.size)
+    ovf, oidx[obins] = fold_lists(obins)
     target = np.zeros(n, dtype=np.int64)
     tl = np.where(rank < 2, rank * FSTRIDE + sb, 2 * FSTRIDE + 2 * oidx[sb] + (rank - 2))
     target[order] = tl
@@ -289,7 +289,6 @@ def scatter_table(bins, gr, gi):
     rec = np.zeros((n, 2), dtype=np.int32)
     rec[:, 0] = target | (mode << 30)
     rec[:, 1] = _bits(gr)
-    ovf = fold_lists(obins)
     return rec, ovf
 
 
@@ -302,16 +301,21 @@ def inverse_column_wg(col):
 
 
 def fold_lists(obins):
-    """Per inverse-column workgroup list of (bin | overflow index << 16)."""
+    """Per inverse-column workgroup list of (bin | overflow index << 16), and
+    the overflow index of every bin of obins. Entry e of list w has index
+    w FOLD_PER_WG + e, so the pass can load an entry's slots before the entry
+    itself has arrived (it takes any other index too, one load later)."""
     lists = [[] for _ in range(INV_WGS)]
-    for k, b in enumerate(np.asarray(obins).tolist()):
+    index = np.zeros(len(obins), dtype=np.int64)
+    for i, b in enumerate(np.asarray(obins).tolist()):
         w = 0 if b == L else inverse_column_wg(b & 255)
-        lists[w].append(b | (k << 16))
+        assert len(lists[w]) < FOLD_PER_WG, "fold list overflow"
+        index[i] = w * FOLD_PER_WG + len(lists[w])
+        lists[w].append(b | (int(index[i]) << 16))
     out = np.full((INV_WGS, FOLD_PER_WG), -1, dtype=np.int64)
     for w, lst in enumerate(lists):
-        assert len(lst) <= FOLD_PER_WG, "fold list overflow"
         out[w, :len(lst)] = lst
-    return out.astype(np.int32).reshape(-1)
+    return out.astype(np.int32).reshape(-1), index
 
 
 def check_tasks(tasks, ncoef, bands, points=POINTS_PER_TASK):
