@@ -40,8 +40,10 @@ static_assert(kAnalysisChunk == 128 && kAnalysisChunkMinBatch == 256, "chunk con
 // SlicedCQT's coefficients go to a new buffer each call, and streaming both
 // their ends pays earlier: 120 slices 144.4 / 139.2, 128 153.6 / 145.1, 160
 // 212.9 / 188.9, 224 296.4 / 262.3 (its analysis alone 57.6 / 58.6 at 120,
-// 116.2 / 100.9 at 224); its signals are read twice (the overlap) and its
-// slice buffer is read again by the overlap-add, so those are not streamed.
+// 116.2 / 100.9 at 224), and so does its output from kStreamYMinBatch on:
+// 120 slices 137.6 / 135.7, 160 184.3 / 178.3, 224 246.4 / 239.2, its inverse
+// alone at 512 304.4 / 292.1. Its signals are read twice (the overlap), so those
+// are not streamed.
 constexpr int64_t kStreamXMinBatch = 124;
 constexpr int64_t kStreamYMinBatch = 105;
 constexpr int64_t kStreamCoefInMinBatch = 140;

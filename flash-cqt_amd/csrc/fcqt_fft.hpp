@@ -93,6 +93,17 @@ __device__ __forceinline__ void store_out(float* p, float v) {
         *p = v;
 }
 
+// A pair of samples at any 4-byte alignment (rows of odd length), one 8-byte
+// store or load.
+typedef float vec2f_a4 __attribute__((ext_vector_type(2), aligned(4)));
+
+template <Store S>
+__device__ __forceinline__ void store_pair(float* p, float2 v) {
+    const vec2f_a4 a = {v.x, v.y};
+    if constexpr (S == Store::kStream) __builtin_nontemporal_store(a, reinterpret_cast<vec2f_a4*>(p));
+    else *reinterpret_cast<vec2f_a4*>(p) = a;
+}
+
 template <bool STREAM>
 __device__ __forceinline__ float2 load_in(const float2* p) {
     if constexpr (STREAM) {

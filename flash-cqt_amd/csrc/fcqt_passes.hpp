@@ -460,9 +460,9 @@ __device__ __forceinline__ void row_inv_tile(const int b, const int rg, const fl
 
 // The inverse row pass over consecutive slices of a SlicedCQT signal with the
 // overlap-add in its store: one row tile (rows rg RPW ..) of the hops h0 ..
-// h1 - 1 of a signal of S slices, hop h being the output samples [2H h,
+// h1 - 1 of a signal of nslices slices, hop h being the output samples [2H h,
 // 2H (h + 1)) below `length`, the sum of slice h's second half and slice
-// h + 1's first half (slice S - 1's second half alone in the last hop). in and
+// h + 1's first half (the last slice's second half alone in the last hop). in and
 // orow are the signal's first work row and output row.
 //
 // A thread's 16 sample pairs of a slice lie at j = lane + 4096 u, lane = 2 (kk1 +
@@ -475,10 +475,8 @@ __device__ __forceinline__ void row_inv_tile(const int b, const int rg, const fl
 // the signal (its second half), so a tile of k hops costs k + 1 slices; the next
 // slice's rows are loaded while this one is transformed. The sums are
 // k_overlap_add's: (0 + a) + b of the rounded products k_row_inv stores.
-// PAIR: the rows of the output are 8-byte aligned, so a pair is one 8-byte
-// store (its second sample alone may lie past the end).
-template <int RPW, bool PAIR>
-__device__ __forceinline__ void row_inv_ola_tile(const int rg, const int h0, const int h1, const int S,
+template <int RPW, Store S>
+__device__ __forceinline__ void row_inv_ola_tile(const int rg, const int h0, const int h1, const int nslices,
                                                  const long length, const float2* __restrict__ in,
                                                  float* __restrict__ orow, const float2* __restrict__ tws,
                                                  float2* lds, const int tid = threadIdx.x) {
@@ -493,7 +491,7 @@ __device__ __forceinline__ void row_inv_ola_tile(const int rg, const int h0, con
     const int lane = 2 * (rg * RPW + (tid & (RPW - 1)) + 128 * kg);
     constexpr float sc = 0.5f / (float)kL;     // 1/L of the inverse, 1/2 of the retangle
     load_tw2_lds<256>(tw2, tws, tid, 16 * RPW);
-    const int last = min(h1, S - 1);           // the last slice this tile needs
+    const int last = min(h1, nslices - 1);     // the last slice this tile needs
     float2 v[16], next[16], carry[8];
 #pragma unroll
     for (int r = 0; r < 16; ++r) next[r] = row[(long)h0 * kL + 16 * r];
@@ -519,23 +517,20 @@ __device__ __forceinline__ void row_inv_ola_tile(const int rg, const int h0, con
             asm volatile("" : "+v"(v0), "+v"(v1), "+v"(w0), "+v"(w1));    // the rounded products
             if (s > h0) {
                 const float2 z = make_float2(carry[i].x + v0, carry[i].y + v1);
-                if (PAIR && room >= 4096 * i + 2) *reinterpret_cast<float2*>(o + 4096 * i) = z;
-                else {
-                    if (room > 4096 * i) o[4096 * i] = z.x;
-                    if (room > 4096 * i + 1) o[4096 * i + 1] = z.y;
-                }
+                if (room >= 4096 * i + 2) store_pair<S>(o + 4096 * i, z);
+                else if (room == 4096 * i + 1) o[4096 * i] = z.x;
             }
             carry[i] = make_float2(0.0f + w0, 0.0f + w1);
         }
         if (s == last) break;
         __syncthreads();                       // every pair read before the next slice overwrites the rows
     }
-    if (h1 == S) {                             // the signal's last hop has no second slice
+    if (h1 == nslices) {                             // the signal's last hop has no second slice
         const long p = 2l * kQuarter * last + lane;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            if (p + 4096 * i < length) orow[p + 4096 * i] = carry[i].x;
-            if (p + 4096 * i + 1 < length) orow[p + 4096 * i + 1] = carry[i].y;
+            if (p + 4096 * i + 1 < length) store_pair<S>(orow + p + 4096 * i, carry[i]);
+            else if (p + 4096 * i < length) orow[p + 4096 * i] = carry[i].x;
         }
     }
 }
@@ -544,8 +539,7 @@ __device__ __forceinline__ void row_inv_ola_tile(const int rg, const int h0, con
 // its store (k_stream_overlap's sums: out[p] = tail[p] + first half, tail[p] =
 // second half, emit = false: tail only). A thread holds both halves of the same
 // positions p (row_inv_ola_tile's runs), so it alone reads and replaces them.
-// PAIR: tail and out are 8-byte aligned.
-template <int RPW, bool PAIR>
+template <int RPW>
 __device__ __forceinline__ void row_inv_stream_tile(const int rg, const bool odd, const bool emit,
                                                     const float2* __restrict__ in, float* __restrict__ tail,
                                                     float* __restrict__ out, const float2* __restrict__ tws,
@@ -558,8 +552,8 @@ __device__ __forceinline__ void row_inv_stream_tile(const int rg, const bool odd
     if (emit) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            if constexpr (PAIR) old[i] = *reinterpret_cast<const float2*>(tail + lane + 4096 * i);
-            else old[i] = make_float2(tail[lane + 4096 * i], tail[lane + 4096 * i + 1]);
+            const vec2f_a4 a = *reinterpret_cast<const vec2f_a4*>(tail + lane + 4096 * i);
+            old[i] = make_float2(a.x, a.y);
         }
     }
     row_fft_to_lds<false, false>(in + (rg * RPW + (tid >> 4)) * 256, lds, lds + RPW * P::US, tid >> 4, tid & 15,
@@ -573,15 +567,8 @@ __device__ __forceinline__ void row_inv_stream_tile(const int rg, const bool odd
         float v0 = a.x * sc, v1 = -a.y * sc;
         asm volatile("" : "+v"(v0), "+v"(v1));    // the rounded products, as k_row_inv stores them
         const float2 z = make_float2(old[i].x + v0, old[i].y + v1), w = make_float2(b.x * sc, -b.y * sc);
-        float* tp = tail + lane + 4096 * i;
-        float* op = out + lane + 4096 * i;
-        if constexpr (PAIR) {
-            if (emit) *reinterpret_cast<float2*>(op) = z;
-            *reinterpret_cast<float2*>(tp) = w;
-        } else {
-            if (emit) op[0] = z.x, op[1] = z.y;
-            tp[0] = w.x, tp[1] = w.y;
-        }
+        if (emit) store_pair<Store::kPlain>(out + lane + 4096 * i, z);
+        store_pair<Store::kPlain>(tail + lane + 4096 * i, w);
     }
 }
 

@@ -132,7 +132,7 @@ static int inv_passes(const float2* f, float2* work, float2* y, const float2* tw
 // The inverse row pass of a whole sliced signal with the overlap-add in its
 // store (row_inv_ola_tile): tiles of `hops` hops of the `nhops` that the output
 // of `length` samples has.
-template <int RPW, bool PAIR>
+template <int RPW, Store ST>
 __global__ __launch_bounds__(16 * RPW) void k_row_inv_ola(const float2* __restrict__ in, float* __restrict__ out,
                                                           const float2* __restrict__ tws, int S, long length,
                                                           int nhops, int hops) {
@@ -143,14 +143,14 @@ __global__ __launch_bounds__(16 * RPW) void k_row_inv_ola(const float2* __restri
     const int r = lg / kWgs;                      // sig * per + hop tile
     const int sig = r / per;
     const int h0 = (r - sig * per) * hops;
-    row_inv_ola_tile<RPW, PAIR>(lg - r * kWgs, h0, min(h0 + hops, nhops), S, length, in + (long)sig * S * kL,
+    row_inv_ola_tile<RPW, ST>(lg - r * kWgs, h0, min(h0 + hops, nhops), S, length, in + (long)sig * S * kL,
                                 out + (long)sig * length, tws, lds);
 }
 
 // The inverse row pass of one streamed slice per signal (row_inv_stream_tile).
 // At 8 signals it took the row pass and k_stream_overlap 4.0 + 2.6 us and a
 // launch between them.
-template <int RPW, bool PAIR>
+template <int RPW>
 __global__ __launch_bounds__(16 * RPW) void k_row_inv_stream(const float2* __restrict__ in, float* __restrict__ tail,
                                                              float* __restrict__ out,
                                                              const float2* __restrict__ tws, int odd, int emit) {
@@ -158,7 +158,7 @@ __global__ __launch_bounds__(16 * RPW) void k_row_inv_stream(const float2* __res
     __shared__ float2 lds[row_lds<RPW>()];
     const int lg = xcd_remap((int)blockIdx.x, (int)gridDim.x);
     const int b = lg / kWgs;
-    row_inv_stream_tile<RPW, PAIR>(lg - b * kWgs, odd, emit, in + (long)b * kL, tail + (long)b * 2 * kQuarter,
+    row_inv_stream_tile<RPW>(lg - b * kWgs, odd, emit, in + (long)b * kL, tail + (long)b * 2 * kQuarter,
                                    out + (long)b * 2 * kQuarter, tws, lds);
 }
 
@@ -187,22 +187,22 @@ static int col_inv_pass(const float2* f, float2* work, const float2* twp, const 
 // slices in two read-add-store launches 313.3 us at 511 hops.
 static int64_t ola_hops(int64_t total) { return total < 160 ? 1 : (total < 320 ? 2 : 4); }
 
-template <int RPW, bool PAIR>
+template <int RPW, Store ST>
 static int row_inv_ola_pass(const float2* work, float* out, const float2* tws, int64_t nsig, int64_t S, int64_t length,
                             hipStream_t stream) {
     constexpr int64_t kWgs = 128 / RPW, kHop = 2 * kQuarter;
     const int64_t nhops = (length + kHop - 1) / kHop;
     const int64_t hops = ola_hops(nsig * nhops);
     const int64_t grid = nsig * ((nhops + hops - 1) / hops) * kWgs;
-    hipLaunchKernelGGL((k_row_inv_ola<RPW, PAIR>), dim3((unsigned)grid), dim3(16 * RPW), 0, stream, work, out, tws,
+    hipLaunchKernelGGL((k_row_inv_ola<RPW, ST>), dim3((unsigned)grid), dim3(16 * RPW), 0, stream, work, out, tws,
                        (int)S, (long)length, (int)nhops, (int)hops);
     return launch_status();
 }
 
-template <int RPW, bool PAIR>
+template <int RPW>
 static int row_inv_stream_pass(const float2* work, float* tail, float* out, const float2* tws, int64_t nsig,
                                int64_t slice, hipStream_t stream) {
-    hipLaunchKernelGGL((k_row_inv_stream<RPW, PAIR>), dim3((unsigned)(nsig * (128 / RPW))), dim3(16 * RPW), 0, stream,
+    hipLaunchKernelGGL((k_row_inv_stream<RPW>), dim3((unsigned)(nsig * (128 / RPW))), dim3(16 * RPW), 0, stream,
                        work, tail, out, tws, (int)(slice & 1), slice > 0 ? 1 : 0);
     return launch_status();
 }
@@ -216,12 +216,9 @@ int stream_inv_passes(const fcqt_tables* tab, const int32_t* ovf, const float* f
                              nsig, stream))
         return e;
     if (!out) out = tail;                         // slice 0 stores no output
-    const bool pair = aligned(tail, 8) && aligned(out, 8);
     if (nsig <= kNarrowMaxBatch)
-        return pair ? row_inv_stream_pass<kRowsNarrow, true>(w2, tail, out, tws, nsig, slice, stream)
-                    : row_inv_stream_pass<kRowsNarrow, false>(w2, tail, out, tws, nsig, slice, stream);
-    return pair ? row_inv_stream_pass<kRowsWide, true>(w2, tail, out, tws, nsig, slice, stream)
-                : row_inv_stream_pass<kRowsWide, false>(w2, tail, out, tws, nsig, slice, stream);
+        return row_inv_stream_pass<kRowsNarrow>(w2, tail, out, tws, nsig, slice, stream);
+    return row_inv_stream_pass<kRowsWide>(w2, tail, out, tws, nsig, slice, stream);
 }
 
 }  // namespace fcqt
@@ -249,12 +246,11 @@ extern "C" int fcqt_sliced_synthesis(const fcqt_tables* tab, const int32_t* scat
                              reinterpret_cast<const float2*>(tab->tw_half), reinterpret_cast<const int*>(ovf), tws,
                              batch, stream))
         return e;
-    const bool pair = (length % 2 == 0 || nsig == 1) && aligned(out, 8);
     if (batch <= kNarrowMaxBatch)
-        return pair ? row_inv_ola_pass<kRowsNarrow, true>(w2, out, tws, nsig, nslices, length, stream)
-                    : row_inv_ola_pass<kRowsNarrow, false>(w2, out, tws, nsig, nslices, length, stream);
-    return pair ? row_inv_ola_pass<kRowsWide, true>(w2, out, tws, nsig, nslices, length, stream)
-                : row_inv_ola_pass<kRowsWide, false>(w2, out, tws, nsig, nslices, length, stream);
+        return row_inv_ola_pass<kRowsNarrow, Store::kPlain>(w2, out, tws, nsig, nslices, length, stream);
+    if (batch < kStreamYMinBatch)
+        return row_inv_ola_pass<kRowsWide, Store::kPlain>(w2, out, tws, nsig, nslices, length, stream);
+    return row_inv_ola_pass<kRowsWide, Store::kStream>(w2, out, tws, nsig, nslices, length, stream);
 }
 
 extern "C" int fcqt_packed_fft_fwd(const fcqt_tables* tab, const float* x, float* xs, float* work,
