@@ -15,6 +15,42 @@ __global__ __launch_bounds__(256) void k_fill_zero(float4* __restrict__ p4, long
     if (i < ntail) tail[i] = 0.0f;
 }
 
+// Several buffers in one launch, 8 KiB per workgroup, so that few small ones
+// still spread over the chip (16-byte accesses where both ends allow them).
+// Graphed returns its outputs with it: a B = 1 round trip's planes and signal
+// (1.3 MB) in one launch instead of three copies by the runtime, the whole call
+// 54.1 -> 43.9 us (torch's foreach copy, 64 Ki elements per workgroup, was slower
+// than the three copies).
+constexpr int64_t kCopyPerWg = 8192;
+struct CopyArgs {
+    const char* src[FCQT_COPY_MAX];
+    char* dst[FCQT_COPY_MAX];
+    long bytes[FCQT_COPY_MAX];
+    unsigned first[FCQT_COPY_MAX + 1];   // first workgroup of each buffer
+    int count;
+};
+
+__global__ __launch_bounds__(256) void k_copy_buffers(const CopyArgs a) {
+    int i = 0;
+    while (i + 1 < a.count && blockIdx.x >= a.first[i + 1]) ++i;
+    const char* s = a.src[i];
+    char* d = a.dst[i];
+    const long lo = (long)(blockIdx.x - a.first[i]) * kCopyPerWg;
+    const long hi = min(lo + (long)kCopyPerWg, a.bytes[i]);
+    const uintptr_t both = reinterpret_cast<uintptr_t>(s) | reinterpret_cast<uintptr_t>(d);
+    long done = lo;                      // whole words first, the rest byte by byte
+    if (both % 16 == 0) {
+        for (long k = lo + 16 * threadIdx.x; k + 16 <= hi; k += 4096)
+            *reinterpret_cast<float4*>(d + k) = *reinterpret_cast<const float4*>(s + k);
+        done = lo + (hi - lo) / 16 * 16;
+    } else if (both % 4 == 0) {
+        for (long k = lo + 4 * threadIdx.x; k + 4 <= hi; k += 1024)
+            *reinterpret_cast<unsigned*>(d + k) = *reinterpret_cast<const unsigned*>(s + k);
+        done = lo + (hi - lo) / 4 * 4;
+    }
+    for (long k = done + threadIdx.x; k < hi; k += 256) d[k] = s[k];
+}
+
 }  // namespace fcqt
 
 using namespace fcqt;
@@ -48,6 +84,26 @@ extern "C" int fcqt_fill_zero(float* buf, int64_t n, hipStream_t stream) {
     if (blocks > 4096) blocks = 4096;
     hipLaunchKernelGGL(k_fill_zero, dim3((unsigned)blocks), dim3(256), 0, stream,
                        reinterpret_cast<float4*>(buf), n4, buf + 4 * n4, ntail);
+    return launch_status();
+}
+
+extern "C" int fcqt_copy_buffers(const void* const* src, void* const* dst, const int64_t* bytes, int count,
+                                 hipStream_t stream) {
+    if (!src || !dst || !bytes || count < 1 || count > FCQT_COPY_MAX) return FCQT_EARG;
+    CopyArgs a = {};
+    int64_t wgs = 0;
+    for (int i = 0; i < count; ++i) {
+        if (!src[i] || !dst[i] || bytes[i] < 1 || bytes[i] > (int64_t)1 << 40) return FCQT_EARG;
+        a.src[i] = static_cast<const char*>(src[i]);
+        a.dst[i] = static_cast<char*>(dst[i]);
+        a.bytes[i] = (long)bytes[i];
+        a.first[i] = (unsigned)wgs;
+        wgs += (bytes[i] + kCopyPerWg - 1) / kCopyPerWg;
+        if (wgs > 1 << 23) return FCQT_EARG;         // 64 GiB in all: the grid's limit
+    }
+    a.first[count] = (unsigned)wgs;
+    a.count = count;
+    hipLaunchKernelGGL(k_copy_buffers, dim3((unsigned)wgs), dim3(256), 0, stream, a);
     return launch_status();
 }
 

@@ -174,20 +174,20 @@ bool plain_call() {
            c10::hip::currentStreamCaptureStatusMayInitCtx() == c10::hip::CaptureStatus::None;
 }
 
-// A dense tensor of this engine's GPU and of the given type, no lazy
-// conjugation or negation, no tangent.
-bool plain_tensor(const Engine& e, const Tensor& t, at::ScalarType type) {
+// A strided tensor of the given GPU and type, no lazy conjugation or
+// negation, no tangent.
+bool plain_tensor(const c10::Device& device, const Tensor& t, at::ScalarType type) {
     static const c10::DispatchKeySet odd({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchBatched,
                                           c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::Functionalize,
                                           c10::DispatchKey::Conjugate, c10::DispatchKey::Negative,
                                           c10::DispatchKey::ZeroTensor});
-    return t.defined() && !t.key_set().has_any(odd) && t.layout() == c10::kStrided && t.device() == e.device &&
+    return t.defined() && !t.key_set().has_any(odd) && t.layout() == c10::kStrided && t.device() == device &&
            t.scalar_type() == type && !t._fw_grad(0).defined();
 }
 
 // (octave blocks, side blocks) of x [..., N], or None
 py::object fwd(const Ref& e, const Tensor& x) {
-    if (!plain_call() || !plain_tensor(*e, x, at::kFloat)) return py::none();
+    if (!plain_call() || !plain_tensor(e->device, x, at::kFloat)) return py::none();
     const int64_t dim = x.dim();
     if (dim < 1 || x.size(-1) != FCQT_N || x.numel() == 0 || !x.is_contiguous()) return py::none();
     const bool grad = x.requires_grad() && at::GradMode::is_enabled();
@@ -244,7 +244,7 @@ py::object bwd(const Ref& e, const std::vector<Tensor>& parts) {
     bool grad = false;
     for (size_t i = 0; i < parts.size(); ++i) {
         const Tensor& c = parts[i];
-        if (!plain_tensor(*e, c, at::kComplexFloat) || c.dim() != dim || c.sizes().slice(0, dim - 2) != lead ||
+        if (!plain_tensor(e->device, c, at::kComplexFloat) || c.dim() != dim || c.sizes().slice(0, dim - 2) != lead ||
             c.size(-2) != e->groups[i].bands || c.size(-1) != e->groups[i].M)
             return py::none();
         grad = grad || c.requires_grad();
@@ -280,12 +280,37 @@ py::object guarded(F f, const A&... a) {
     }
 }
 
+// Copies of the tensors (t.clone() each) with one launch of fcqt_copy_buffers, or
+// None where one of them is not a plain dense tensor of the current GPU.
+py::object clones(const std::vector<Tensor>& ts, int64_t copy_fn) {
+    if (ts.empty() || ts.size() > FCQT_COPY_MAX || !plain_call()) return py::none();
+    const c10::Device device(c10::kCUDA, c10::hip::current_device());
+    const void* src[FCQT_COPY_MAX];
+    void* dst[FCQT_COPY_MAX];
+    int64_t bytes[FCQT_COPY_MAX];
+    for (const Tensor& t : ts)
+        if (!plain_tensor(device, t, t.scalar_type()) || !t.is_non_overlapping_and_dense() || t.numel() == 0)
+            return py::none();
+    std::vector<Tensor> out;
+    for (size_t i = 0; i < ts.size(); ++i) {
+        out.push_back(at::empty_like(ts[i]));
+        src[i] = ts[i].data_ptr();
+        dst[i] = out[i].data_ptr();
+        bytes[i] = (int64_t)ts[i].nbytes();
+    }
+    if (int s = reinterpret_cast<decltype(&fcqt_copy_buffers)>(copy_fn)(
+            src, dst, bytes, (int)ts.size(), c10::hip::getCurrentHIPStream(device.index()).stream()))
+        raise_native(s, "copy_buffers");
+    return py::cast(out);
+}
+
 const void* address(int64_t p) { return reinterpret_cast<const void*>(p); }
 
 }  // namespace
 
 PYBIND11_MODULE(_fcqt_torch, m) {
     // [t.as_strided(size, stride, offset) for size, stride, offset in args]
+    m.def("clones", [](const std::vector<Tensor>& ts, int64_t copy_fn) { return guarded(clones, ts, copy_fn); });
     m.def("strided_views", [](const Tensor& t, const std::vector<std::tuple<std::vector<int64_t>, std::vector<int64_t>,
                                                                             int64_t>>& args) {
         std::vector<Tensor> out;

@@ -29,7 +29,7 @@ INTERLEAVED = 1
 #: every symbol include/flashcqt.h declares
 EXPORTS = ("fcqt_abi_version", "fcqt_status_string", "fcqt_last_hip_error",
            "fcqt_packed_fft_fwd", "fcqt_route_bands", "fcqt_scatter_bands",
-           "fcqt_packed_fft_inv", "fcqt_analysis", "fcqt_synthesis", "fcqt_fill_zero",
+           "fcqt_packed_fft_inv", "fcqt_analysis", "fcqt_synthesis", "fcqt_fill_zero", "fcqt_copy_buffers",
            "fcqt_slice_fft_fwd", "fcqt_route_bands_sliced", "fcqt_scatter_bands_sliced",
            "fcqt_overlap_add", "fcqt_stream_overlap", "fcqt_image_check", "fcqt_tables_upload",
            "fcqt_workspace_sizes", "fcqt_analysis_static", "fcqt_persist_analysis", "fcqt_persist_synthesis",
@@ -130,6 +130,7 @@ def _open(path):
         "fcqt_analysis": ([T, P, P, P, P, ctypes.c_int, P, P, I64, S], ctypes.c_int),
         "fcqt_synthesis": ([T, P, P, P, P, ctypes.c_int, P, P, P, I64, S], ctypes.c_int),
         "fcqt_fill_zero": ([P, I64, S], ctypes.c_int),
+        "fcqt_copy_buffers": ([P, P, P, ctypes.c_int, S], ctypes.c_int),
         "fcqt_slice_fft_fwd": ([T, P, I64, P, I64, I64, I64, I64, P, P, S], ctypes.c_int),
         "fcqt_route_bands_sliced": ([T, P, P, P, P, I64, I64, I64, S], ctypes.c_int),
         "fcqt_sliced_analysis": ([T, P, P, P, I64, P, I64, I64, P, P, P, S], ctypes.c_int),

@@ -12,7 +12,11 @@ device are converted by the copy); a shape mismatch raises instead of being
 broadcast into the recorded buffers.
 Reference surface: graphed.py:35-57.
 """
+import ctypes
+
 import torch
+
+from . import _native
 
 
 def _leaves(t):
@@ -74,4 +78,17 @@ class Graphed:
         for dst, src in zip(self._slots, given):
             dst.copy_(src)
         self.graph.replay()
-        return _map(self._out, lambda t: t.clone())
+        return self._clones()
+
+    def _clones(self):
+        """The recorded outputs as tensors of their own: one launch where the
+        host glue takes them, else one clone each."""
+        glue = _native.load_glue()
+        outs = list(_leaves(self._out))
+        new = None
+        if glue is not None and all(type(t) is torch.Tensor for t in outs):
+            new = glue.clones(outs, ctypes.cast(_native.load().fcqt_copy_buffers, ctypes.c_void_p).value)
+        if new is None:
+            return _map(self._out, lambda t: t.clone())
+        new = iter(new)
+        return _map(self._out, lambda t: next(new))

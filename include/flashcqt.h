@@ -450,6 +450,13 @@ int fcqt_stream_synthesis(const fcqt_tables* tab, const int32_t* scat, const int
 /* Zero n floats with a fill kernel (graph-capture safe, no hipMemsetAsync). */
 int fcqt_fill_zero(float* buf, int64_t n, hipStream_t stream);
 
+/* Copy bytes[i] bytes (>= 1) from src[i] to dst[i] for i < count <=
+ * FCQT_COPY_MAX with one kernel: the outputs of a replayed graph into buffers of
+ * their own. The three arrays are host memory, read before the call returns; the
+ * buffers are device memory of any alignment and do not overlap. */
+#define FCQT_COPY_MAX 16
+int fcqt_copy_buffers(const void* const* src, void* const* dst, const int64_t* bytes, int count, hipStream_t stream);
+
 #ifdef __cplusplus
 }
 #endif
