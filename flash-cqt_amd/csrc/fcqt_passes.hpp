@@ -158,7 +158,7 @@ __device__ __forceinline__ void col_fwd_tile(const int b, const int cg, const fl
     } else {
         const float2* xb = in + (long)b * kL;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) v[r] = load_in<STREAM>(xb + 256 * (t + 8 * r) + n2);
+        for (int r = 0; r < 16; ++r) v[r] = load_in<STREAM>(xb + (256 * (t + 8 * r) + n2));
     }
     // every twiddle this thread needs, in flight with the data
     load_tw2_lds<128>(tw2, tws, tid, 8 * CPW);
@@ -366,7 +366,7 @@ __device__ __forceinline__ void row_fft_to_lds(const float2* __restrict__ yrow, 
     using P = Plan<256>;
     float2 v[16];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) v[r] = load_in<STREAM>(yrow + t + 16 * r);
+    for (int r = 0; r < 16; ++r) v[r] = load_in<STREAM>(yrow + (t + 16 * r));
     load_tw2_lds<256>(tw2, tws, tid, nthreads);
     if constexpr (HOLD) {
         asm volatile("" : "+v"(vhold->x), "+v"(vhold->y));
