@@ -301,8 +301,8 @@ class SlicedCQT:
     def _views(coef, args):
         """as_strided views of one coefficient buffer, in one call where the
         host glue is built."""
-        glue = _native.load_glue()
-        if glue is not None and not torch.compiler.is_compiling():
+        glue = None if torch.compiler.is_compiling() else _native.load_glue()
+        if glue is not None:
             return glue.strided_views(coef, args)
         return [coef.as_strided(*a) for a in args]
 
