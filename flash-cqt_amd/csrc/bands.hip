@@ -97,7 +97,8 @@ static void launch_route(int64_t ntasks, int64_t batch, hipStream_t stream, cons
                       kBandSliceMajorMinBatch <= kBandWriteThroughMaxBatch,
                   "batch ranges: plain task-major, write-through task-major, write-through slice-major, "
                   "plain slice-major");
-    if (total >= (LAYOUT == kSliced ? kStreamSlicedCoefMinBatch : kStreamCoefOutMinBatch))
+    if (total >= (LAYOUT == kSliced ? kStreamSlicedCoefMinBatch
+                  : LAYOUT == FCQT_INTERLEAVED ? kStreamNewCoefOutMinBatch : kStreamCoefOutMinBatch))
         hipLaunchKernelGGL((k_route_bands<LAYOUT, Store::kStream, true>), grid, dim3(kBandThreads), 0, stream, xs, cre,
                            cim, rec, tasks, (int)batch, ncoef, sm, tws, (int)ntasks);
     else if (batch > kBandWriteThroughMaxBatch)

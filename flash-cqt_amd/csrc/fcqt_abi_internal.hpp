@@ -37,8 +37,12 @@ static_assert(kAnalysisChunk == 128 && kAnalysisChunkMinBatch == 256, "chunk con
 //           alone 256 134.7 / 117.4, 512 271.8 / 221.2
 //   W read by the row pass (with those): B = 192 194.7 / 194.9,
 //           256 266.1 / 257.7, 512 550 / 518
-// SlicedCQT's coefficients go to a new buffer each call, and streaming both
-// their ends pays earlier: 120 slices 144.4 / 139.2, 128 153.6 / 145.1, 160
+// TrainableCQT's coefficients (interleaved) go to a new buffer each call, so
+// nothing in the caches is there for them: written past the caches from 140
+// slices on, training steps at 144 / 160 / 176 slices 404 / 436 / 469 -> 386 / 418 /
+// 460 us and round trips without gradients 153.5 / 167.7 / 183.1 -> 151.8 / 163.9 /
+// 177.7 (from 105 on steps gain as much, but round trips lose 4 us up to 127).
+// So do SlicedCQT's, and streaming both their ends pays earlier: 120 slices 144.4 / 139.2, 128 153.6 / 145.1, 160
 // 212.9 / 188.9, 224 296.4 / 262.3 (its analysis alone 57.6 / 58.6 at 120,
 // 116.2 / 100.9 at 224), and so does its output from kStreamYMinBatch on:
 // 120 slices 137.6 / 135.7, 160 184.3 / 178.3, 224 246.4 / 239.2, its inverse
@@ -48,6 +52,7 @@ constexpr int64_t kStreamXMinBatch = 124;
 constexpr int64_t kStreamYMinBatch = 105;
 constexpr int64_t kStreamCoefInMinBatch = 140;
 constexpr int64_t kStreamCoefOutMinBatch = 192;
+constexpr int64_t kStreamNewCoefOutMinBatch = 140;
 constexpr int64_t kStreamWMinBatch = 192;
 constexpr int64_t kStreamSlicedCoefMinBatch = 105;
 
