@@ -120,6 +120,11 @@ class TrainableCQT:
             if c._base is not base or c.data_ptr() != ptr + 8 * off or c.stride()[-2:] != (M, 1) \
                     or c.shape[-2:] != (b, M):
                 return None
+            row = self.ncoef               # strides of the leading dimensions, last first: the slices in order
+            for size, stride in zip(c.shape[-3::-1], c.stride()[-3::-1]):
+                if size != 1 and stride != row:
+                    return None
+                row *= size
         return base
 
     def bwd(self, blocks, side=None):

@@ -115,3 +115,30 @@ def test_glue_step_in_a_graph_and_from_threads(pair):
     torch.cuda.synchronize()
     with ThreadPoolExecutor(4) as pool:        # on one stream
         assert all(torch.equal(y, want) for y in pool.map(lambda i: t.bwd(*t.fwd(x)), range(16)))
+
+
+@pytest.fixture(scope="module")
+def cqt():
+    from flash_cqt import OctCQT
+    return OctCQT([3, 4, 2], [8, 16, 32], fs=44100, audio_len=N, device="cuda:0")
+
+
+def _engine(cqt, path):
+    from flash_cqt.trainable import TrainableCQT
+    t = TrainableCQT(cqt, "cuda:0")
+    if path == "python":
+        t._glue = None
+    return t
+
+
+@pytest.mark.parametrize("path", ["glue", "python"])
+def test_turned_views_on_a_first_call_and_later(cqt, path):
+    """Slices in the order given, whichever path takes the call: on buffers that
+    the engine has released (a first call), and again with them there."""
+    t = _engine(cqt, path)
+    blocks, side = t.fwd(_x(2, 3))
+    want = t.bwd(blocks, side).transpose(0, 1)
+    for cold in (True, False):
+        if cold:
+            t.f.release_workspace()
+        assert torch.equal(t.bwd([c.transpose(0, 1) for c in blocks], [c.transpose(0, 1) for c in side]), want)

@@ -1,0 +1,36 @@
+"""Host logic of TrainableCQT that needs no GPU: which block tensors bwd may
+read as the coefficient buffer that they are views of."""
+import pytest
+import torch
+
+GSPEC = [(2, 4, 0), (1, 8, 8), (1, 4, 16)]
+NCOEF = 20
+
+
+@pytest.fixture()
+def engine():
+    from flash_cqt.trainable import TrainableCQT
+    t = TrainableCQT.__new__(TrainableCQT)
+    t.dev, t.gspec, t.ncoef, t.ngroups = torch.device("cpu"), GSPEC, NCOEF, 2
+    return t
+
+
+def _kc(rows=6):
+    return torch.randn(rows, NCOEF, dtype=torch.complex64, generator=torch.Generator().manual_seed(rows))
+
+
+def _views(kc, *lead):
+    return [kc.narrow(1, off, b * M).view(*lead, b, M) for b, M, off in GSPEC]
+
+
+@pytest.mark.parametrize("lead", [(6,), (2, 3), (1, 6), (6, 1), (3, 1, 2)])
+def test_fwd_views_are_read_as_their_buffer(engine, lead):
+    kc = _kc()
+    assert engine._base_of(_views(kc, *lead), 6) is kc
+
+
+@pytest.mark.parametrize("lead,turn", [((2, 3), (1, 0)), ((3, 2), (1, 0)), ((3, 1, 2), (2, 1, 0)), ((1, 2, 3), (0, 2, 1))])
+def test_views_in_another_slice_order_are_not_the_buffer(engine, lead, turn):
+    n = len(lead)
+    parts = [c.permute(*turn, n, n + 1) for c in _views(_kc(), *lead)]
+    assert engine._base_of(parts, 6) is None
