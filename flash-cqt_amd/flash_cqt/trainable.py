@@ -112,7 +112,7 @@ class TrainableCQT:
         """The [B, ncoef] complex64 buffer whose consecutive group views the
         parts are (as fwd returns them), else None."""
         base = parts[0]._base
-        if base is None or base.device != self.dev or base.dtype != torch.complex64 \
+        if len(parts) != len(self.gspec) or base is None or base.device != self.dev or base.dtype != torch.complex64 \
                 or base.shape != (B, self.ncoef) or not base.is_contiguous():
             return None
         ptr = base.data_ptr()
@@ -125,6 +125,8 @@ class TrainableCQT:
                 if size != 1 and stride != row:
                     return None
                 row *= size
+            if row != B * self.ncoef:
+                return None
         return base
 
     def bwd(self, blocks, side=None):

@@ -142,3 +142,15 @@ def test_turned_views_on_a_first_call_and_later(cqt, path):
         if cold:
             t.f.release_workspace()
         assert torch.equal(t.bwd([c.transpose(0, 1) for c in blocks], [c.transpose(0, 1) for c in side]), want)
+
+
+@pytest.mark.parametrize("path", ["glue", "python"])
+def test_blocks_that_are_missing_or_cropped_are_refused(cqt, path):
+    t = _engine(cqt, path)
+    blocks, side = t.fwd(_x(4))
+    with pytest.raises(ValueError):
+        t.bwd(blocks, [])
+    with pytest.raises(ValueError):
+        t.bwd(blocks[:-1], side)
+    with pytest.raises(ValueError):
+        t.bwd([*blocks[:-1], blocks[-1][:2]], side)

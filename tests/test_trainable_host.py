@@ -34,3 +34,12 @@ def test_views_in_another_slice_order_are_not_the_buffer(engine, lead, turn):
     n = len(lead)
     parts = [c.permute(*turn, n, n + 1) for c in _views(_kc(), *lead)]
     assert engine._base_of(parts, 6) is None
+
+
+def test_part_of_the_views_is_not_the_buffer(engine):
+    """Fewer slices in one block, or fewer blocks, than the buffer holds."""
+    parts = _views(_kc(), 6)
+    for i in range(3):
+        assert engine._base_of([c[:2] if j == i else c for j, c in enumerate(parts)], 6) is None
+    assert engine._base_of(parts[:2], 6) is None
+    assert engine._base_of(parts[:2] + [parts[1], parts[2]], 6) is None
