@@ -316,6 +316,7 @@ class SlicedCQT:
                 and base.numel() == nsig * S * f.ncoef and base.device == f.dev and base.is_contiguous():
             ptr = base.data_ptr()
             if all(p._base is base and p.is_contiguous() and p.data_ptr() == ptr + 8 * nsig * S * off
+                   and not p.is_conj() and not p.is_neg()
                    for p, (_, _, off) in zip(parts, f.gspec)):
                 return base
         coef = torch.zeros(nsig * S * f.ncoef, dtype=torch.complex64, device=f.dev)

@@ -102,7 +102,7 @@ class TrainableCQT:
             raise ValueError(f"x is on {xf.device}, engine on {self.dev}")
         if xf.shape[0] < 1:
             raise ValueError("x needs at least one slice")
-        kc = _Analysis.apply(xf.contiguous(), self)
+        kc = _Analysis.apply(xf.resolve_neg().contiguous(), self)
         # one narrow per group (not a multi-output split): the blocks stay
         # single views, which autograd lets a caller modify in place
         views = [kc.narrow(1, off, b * M).view(*lead, b, M) for b, M, off in self.gspec]
@@ -118,7 +118,7 @@ class TrainableCQT:
         ptr = base.data_ptr()
         for c, (b, M, off) in zip(parts, self.gspec):
             if c._base is not base or c.data_ptr() != ptr + 8 * off or c.stride()[-2:] != (M, 1) \
-                    or c.shape[-2:] != (b, M):
+                    or c.shape[-2:] != (b, M) or c.is_conj() or c.is_neg():
                 return None
             row = self.ncoef               # strides of the leading dimensions, last first: the slices in order
             for size, stride in zip(c.shape[-3::-1], c.stride()[-3::-1]):
@@ -156,7 +156,7 @@ class TrainableCQT:
             raise ValueError(f"blocks carry {flat.shape[-1]} coefficients, expected {self.ncoef}")
         if flat.device != self.dev:
             raise ValueError(f"blocks are on {flat.device}, engine on {self.dev}")
-        return _Synthesis.apply(flat.contiguous(), self).reshape(*lead, N)
+        return _Synthesis.apply(flat.resolve_conj().contiguous(), self).reshape(*lead, N)
 
 
 class _Analysis(torch.autograd.Function):
@@ -167,7 +167,7 @@ class _Analysis(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, gk):
-        return ctx.eng._adj_analysis(gk.to(torch.complex64).contiguous()), None
+        return ctx.eng._adj_analysis(gk.to(torch.complex64).resolve_conj().contiguous()), None
 
 
 class _Synthesis(torch.autograd.Function):
@@ -178,4 +178,4 @@ class _Synthesis(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, gy):
-        return ctx.eng._adj_synthesis(gy.float().contiguous()), None
+        return ctx.eng._adj_synthesis(gy.float().resolve_neg().contiguous()), None

@@ -154,3 +154,22 @@ def test_blocks_that_are_missing_or_cropped_are_refused(cqt, path):
         t.bwd(blocks[:-1], side)
     with pytest.raises(ValueError):
         t.bwd([*blocks[:-1], blocks[-1][:2]], side)
+
+
+@pytest.mark.parametrize("path", ["glue", "python"])
+def test_conjugated_blocks_are_conjugated(cqt, path):
+    """Lazily conjugated views of fwd's buffer, against blocks of their own."""
+    t = _engine(cqt, path)
+    blocks, side = t.fwd(_x(3))
+    own = lambda parts: [c.conj().resolve_conj() for c in parts]  # noqa: E731
+    want = t.bwd(own(blocks), own(side))
+    assert torch.equal(t.bwd([c.conj() for c in blocks], [c.conj() for c in side]), want)
+    assert torch.equal(t.bwd([c.conj() for c in blocks], own(side)), want)
+
+
+def test_sliced_conjugated_blocks_are_conjugated():
+    from flash_cqt import SlicedCQT
+    s = SlicedCQT(fs=44100, device="cuda:0")
+    blocks, side = s.fwd(_x(1, 2))
+    own = lambda parts: [c.conj().resolve_conj() for c in parts]  # noqa: E731
+    assert torch.equal(s.bwd([c.conj() for c in blocks], [c.conj() for c in side]), s.bwd(own(blocks), own(side)))

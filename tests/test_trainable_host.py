@@ -43,3 +43,23 @@ def test_part_of_the_views_is_not_the_buffer(engine):
         assert engine._base_of([c[:2] if j == i else c for j, c in enumerate(parts)], 6) is None
     assert engine._base_of(parts[:2], 6) is None
     assert engine._base_of(parts[:2] + [parts[1], parts[2]], 6) is None
+
+
+def test_conjugated_views_are_not_the_buffer(engine):
+    """conj() is a view with the buffer's address and strides and a flag."""
+    parts = _views(_kc(), 6)
+    for i in range(3):
+        assert engine._base_of([c.conj() if j == i else c for j, c in enumerate(parts)], 6) is None
+
+
+def test_sliced_conjugated_views_are_not_the_buffer():
+    import types
+    from flash_cqt.sliced import SlicedCQT
+    s = SlicedCQT.__new__(SlicedCQT)
+    f = types.SimpleNamespace(gspec=GSPEC, ncoef=NCOEF, dev=torch.device("cpu"))
+    coef = _kc(6).flatten().clone()
+    views = [coef[6 * off:6 * (off + b * M)].view(1, 3, b, 2 * M) for b, M, off in GSPEC]
+    for i in range(3):
+        turned = [c.conj() if j == i else c for j, c in enumerate(views)]
+        got = s._block_buffer(f, turned[:2], turned[2:], 3, 2)
+        assert got is not coef and torch.equal(got, torch.cat([c.flatten().resolve_conj() for c in turned]))
