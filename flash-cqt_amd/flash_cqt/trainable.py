@@ -110,13 +110,18 @@ class TrainableCQT:
 
     def _base_of(self, parts, B):
         """The [B, ncoef] complex64 buffer whose consecutive group views the
-        parts are (as fwd returns them), else None."""
+        parts are (as fwd returns them), else None. A part that is a leaf of
+        its own, or whose gradient is wanted where the buffer's is not, is no
+        such view: its gradient would go past it."""
         base = parts[0]._base
         if len(parts) != len(self.gspec) or base is None or base.device != self.dev or base.dtype != torch.complex64 \
                 or base.shape != (B, self.ncoef) or not base.is_contiguous():
             return None
         ptr = base.data_ptr()
+        grad = torch.is_grad_enabled()
         for c, (b, M, off) in zip(parts, self.gspec):
+            if grad and (c.requires_grad != base.requires_grad or (c.requires_grad and c.is_leaf)):
+                return None
             if c._base is not base or c.data_ptr() != ptr + 8 * off or c.stride()[-2:] != (M, 1) \
                     or c.shape[-2:] != (b, M) or c.is_conj() or c.is_neg():
                 return None

@@ -173,3 +173,20 @@ def test_sliced_conjugated_blocks_are_conjugated():
     blocks, side = s.fwd(_x(1, 2))
     own = lambda parts: [c.conj().resolve_conj() for c in parts]  # noqa: E731
     assert torch.equal(s.bwd([c.conj() for c in blocks], [c.conj() for c in side]), s.bwd(own(blocks), own(side)))
+
+
+@pytest.mark.parametrize("path", ["glue", "python"])
+def test_blocks_made_leaves_get_their_gradients(cqt, path):
+    """Coefficients of a call without gradients, then optimised themselves."""
+    t = _engine(cqt, path)
+    x = _x(3)
+
+    def gradients(keep):
+        with torch.no_grad():
+            blocks, side = t.fwd(x)
+        parts = [keep(c) for c in [*blocks, *side]]
+        for c in parts[1:]:
+            c.requires_grad_(True)
+        y = t.bwd(parts[:len(blocks)], parts[len(blocks):])
+        return torch.autograd.grad((y ** 3).sum(), parts[1:])
+    assert _same(gradients(lambda c: c), gradients(lambda c: c.detach().clone()))

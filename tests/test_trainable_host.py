@@ -63,3 +63,15 @@ def test_sliced_conjugated_views_are_not_the_buffer():
         turned = [c.conj() if j == i else c for j, c in enumerate(views)]
         got = s._block_buffer(f, turned[:2], turned[2:], 3, 2)
         assert got is not coef and torch.equal(got, torch.cat([c.flatten().resolve_conj() for c in turned]))
+
+
+@pytest.mark.parametrize("base_grad", [False, True])
+def test_leaf_views_are_not_the_buffer(engine, base_grad):
+    """Views made without a gradient and then made to want one of their own."""
+    kc = _kc().requires_grad_(base_grad) * 1
+    with torch.no_grad():
+        parts = _views(kc, 6)
+    parts[1].requires_grad_(True)
+    assert engine._base_of(parts, 6) is None
+    with torch.no_grad():
+        assert engine._base_of(parts, 6) is kc
