@@ -52,6 +52,8 @@ struct Engine : torch::CustomClassHolder {
     Tensor X, W, F, FA;
     std::atomic<bool> captured{false};
 
+    // adjoint: with FA, which the gradient of an analysis scatters into (a
+    // synthesis and its gradient use X, W and F alone)
     bool ready(int64_t batch, bool adjoint) {
         std::lock_guard<std::mutex> lock(mu);
         return rows >= batch && (!adjoint || FA.defined());
@@ -245,15 +247,13 @@ py::object bwd(const Ref& e, const std::vector<Tensor>& parts) {
     const auto lead = parts[0].sizes().slice(0, dim - 2);
     int64_t batch = 1;
     for (int64_t d : lead) batch *= d;
-    bool grad = false;
     for (size_t i = 0; i < parts.size(); ++i) {
         const Tensor& c = parts[i];
         if (!plain_tensor(e->device, c, at::kComplexFloat) || c.dim() != dim || c.sizes().slice(0, dim - 2) != lead ||
             c.size(-2) != e->groups[i].bands || c.size(-1) != e->groups[i].M)
             return py::none();
-        grad = grad || c.requires_grad();
     }
-    if (batch < 1 || !e->ready(batch, grad && at::GradMode::is_enabled())) return py::none();
+    if (batch < 1 || !e->ready(batch, false)) return py::none();
     Tensor y;
     {
         py::gil_scoped_release nogil;

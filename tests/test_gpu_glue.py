@@ -190,3 +190,21 @@ def test_blocks_made_leaves_get_their_gradients(cqt, path):
         y = t.bwd(parts[:len(blocks)], parts[len(blocks):])
         return torch.autograd.grad((y ** 3).sum(), parts[1:])
     assert _same(gradients(lambda c: c), gradients(lambda c: c.detach().clone()))
+
+
+def test_ordinary_calls_are_the_glues(cqt):
+    """On a fresh engine, once a call has made its buffers: the directions alone,
+    gains learnt between them (no gradient of the signal), coefficients learnt
+    themselves, and, after one backward pass, training of the signal."""
+    t = _engine(cqt, "glue")
+    x = _x(2, 3)
+    blocks, side = t.fwd(x)
+    assert t._glue.fwd(x) is not None and t._glue.bwd([*blocks, *side]) is not None
+    gains = [torch.full((c.shape[-2], 1), 0.5, device="cuda", requires_grad=True) for c in blocks]
+    leaves = [c.detach().clone().requires_grad_(True) for c in [*blocks, *side]]
+    for parts in ([c * g for c, g in zip(blocks, gains)] + list(side), leaves):
+        y = t._glue.bwd(parts)
+        assert y is not None and y.requires_grad
+    xg = x.clone().requires_grad_(True)
+    t.bwd(*t.fwd(xg)).sum().backward()
+    assert t._glue.fwd(xg) is not None
