@@ -36,7 +36,9 @@ static_assert(kAnalysisChunk == 128 && kAnalysisChunkMinBatch == 256, "chunk con
 //           176 183.9 / 182.8, 200 210.3 / 206.4, 512 592 / 550; the analysis
 //           alone 256 134.7 / 117.4, 512 271.8 / 221.2
 //   W read by the row pass (with those): B = 192 194.7 / 194.9,
-//           256 266.1 / 257.7, 512 550 / 518
+//           256 266.1 / 257.7, 512 550 / 518; not in the 128-slice chunks of
+//           fcqt_sliced_analysis, whose W is in the caches (256 slices 125.5 / 125.8,
+//           320 166.5 / 167.9, 512 263 / 263; layout (4, 3) x (12, 48) 109.1 / 110.5, 146.5 / 148.1, 231 / 229)
 // TrainableCQT's coefficients (interleaved) go to a new buffer each call, so
 // nothing in the caches is there for them: written past the caches from 140
 // slices on, training steps at 144 / 160 / 176 slices 404 / 436 / 469 -> 386 / 418 /
@@ -69,12 +71,6 @@ int check_band_args(const fcqt_tables* tab, const int32_t* rec, const float* cre
 // in packed_fft.hip.
 int packed_fft_inv(const fcqt_tables* tab, const int32_t* ovf, const float* f, float* y, float* work, int64_t batch,
                    bool last, hipStream_t stream);
-
-// fcqt_slice_fft_fwd of one chunk of a call of `total` slices (which sets
-// the cache choices); defined in packed_fft.hip.
-int slice_fft_fwd(const fcqt_tables* tab, const float* sig, int64_t sig_len, const float* window, int64_t nsig,
-                  int64_t nslices, int64_t first, int64_t origin, float* xs, float* work, int64_t total,
-                  hipStream_t stream);
 
 // The inverse passes of one streamed slice per signal with the half-slice
 // overlap-add in the row pass's store (arguments checked by the caller);
