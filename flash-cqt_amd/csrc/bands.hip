@@ -97,8 +97,9 @@ static void launch_route(int64_t ntasks, int64_t batch, hipStream_t stream, cons
                       kBandSliceMajorMinBatch <= kBandWriteThroughMaxBatch,
                   "batch ranges: plain task-major, write-through task-major, write-through slice-major, "
                   "plain slice-major");
-    if (total >= (LAYOUT == kSliced ? kStreamSlicedCoefMinBatch
-                  : LAYOUT == FCQT_INTERLEAVED ? kStreamNewCoefOutMinBatch : kStreamCoefOutMinBatch))
+    const bool past = LAYOUT == kSliced ? stream_sliced_coef(total, ncoef)
+                      : total >= (LAYOUT == FCQT_INTERLEAVED ? kStreamNewCoefOutMinBatch : kStreamCoefOutMinBatch);
+    if (past)
         hipLaunchKernelGGL((k_route_bands<LAYOUT, Store::kStream, true>), grid, dim3(kBandThreads), 0, stream, xs, cre,
                            cim, rec, tasks, (int)batch, ncoef, sm, tws, (int)ntasks);
     else if (batch > kBandWriteThroughMaxBatch)
@@ -120,7 +121,7 @@ static void launch_scatter(int64_t ntasks, int64_t batch, hipStream_t stream, co
                            float* f, const int2* scat, const int4* tasks, long ncoef, const SliceMap& sm,
                            const float2* tws) {
     const dim3 grid((unsigned)(ntasks * batch));
-    if (batch >= (LAYOUT == kSliced ? kStreamSlicedCoefMinBatch : kStreamCoefInMinBatch))
+    if (LAYOUT == kSliced ? stream_sliced_coef(batch, ncoef) : batch >= kStreamCoefInMinBatch)
         hipLaunchKernelGGL((k_scatter_bands<LAYOUT, Store::kPlain, true, true>), grid, dim3(kBandThreads), 0, stream,
                            cre, cim, f, scat, tasks, (int)batch, ncoef, sm, tws, (int)ntasks);
     else if (batch > kBandWriteThroughMaxBatch)

@@ -20,7 +20,7 @@ constexpr int64_t kAnalysisChunk = FCQT_ANALYSIS_CHUNK;
 constexpr int64_t kAnalysisChunkMinBatch = FCQT_ANALYSIS_CHUNK_MIN_BATCH;
 static_assert(kAnalysisChunk == 128 && kAnalysisChunkMinBatch == 256, "chunk constants of the header");
 
-// From these batch sizes on a buffer is written or read past the caches
+// From these sizes on a buffer is written or read past the caches
 // (Store::kStream, load_in<true>). Per slice a round trip touches x, W, X,
 // the coefficients, F and y: 2.7 MB, so about 96 slices fill the 256 MB
 // memory-side cache, and past that a buffer without a nearby reader only
@@ -44,9 +44,13 @@ static_assert(kAnalysisChunk == 128 && kAnalysisChunkMinBatch == 256, "chunk con
 // slices on, training steps at 144 / 160 / 176 slices 404 / 436 / 469 -> 386 / 418 /
 // 460 us and round trips without gradients 153.5 / 167.7 / 183.1 -> 151.8 / 163.9 /
 // 177.7 (from 105 on steps gain as much, but round trips lose 4 us up to 127).
-// So do SlicedCQT's, and streaming both their ends pays earlier: 120 slices 144.4 / 139.2, 128 153.6 / 145.1, 160
-// 212.9 / 188.9, 224 296.4 / 262.3 (its analysis alone 57.6 / 58.6 at 120,
-// 116.2 / 100.9 at 224), and so does its output from kStreamYMinBatch on:
+// So do SlicedCQT's, and streaming both their ends pays earlier, from where a
+// round trip's buffers hold 340 MB (126 slices; 140 in the layout (4, 3) x (12, 48) of
+// 99,072 coefficients against 132,992): round trips at 105 / 112 / 120 / 128 / 136 /
+// 144 / 160 slices 120.5 / 125.1 / 132.7 / 142.6 / 162.0 / 181.3 / 205.3 kept, 126.7 /
+// 130.5 / 137.1 / 142.9 / 160.9 / 165.0 / 176.6 streamed; in that layout 108.2 / 112.5 /
+// 116.8 / 123.5 / 142.4 / 150.8 / 177.4 against 113.3 / 117.5 / 123.3 / 128.6 / 144.9 /
+// 148.9 / 163.8 (two signals of half as many slices alike). So does its output from kStreamYMinBatch on:
 // 120 slices 137.6 / 135.7, 160 184.3 / 178.3, 224 246.4 / 239.2, its inverse
 // alone at 512 304.4 / 292.1. Its signals are read twice (the overlap), so those
 // are not streamed.
@@ -56,7 +60,17 @@ constexpr int64_t kStreamCoefInMinBatch = 140;
 constexpr int64_t kStreamCoefOutMinBatch = 192;
 constexpr int64_t kStreamNewCoefOutMinBatch = 140;
 constexpr int64_t kStreamWMinBatch = 192;
-constexpr int64_t kStreamSlicedCoefMinBatch = 105;
+constexpr int64_t kStreamSlicedCoefBytes = 340000000;
+
+// Bytes of x, W, X and the coefficients, and of a round trip's buffers (F and y
+// too), for a call of `batch` slices.
+inline int64_t analysis_bytes(int64_t batch, int64_t ncoef) { return batch * (4 * FCQT_N + 16 * FCQT_L + 8 * ncoef); }
+inline int64_t round_trip_bytes(int64_t batch, int64_t ncoef) {
+    return analysis_bytes(batch, ncoef) + batch * (8 * FCQT_FROW + 4 * FCQT_N);
+}
+inline bool stream_sliced_coef(int64_t batch, int64_t ncoef) {
+    return round_trip_bytes(batch, ncoef) >= kStreamSlicedCoefBytes;
+}
 
 inline bool aligned(const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
 
