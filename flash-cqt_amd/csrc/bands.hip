@@ -121,7 +121,9 @@ static void launch_scatter(int64_t ntasks, int64_t batch, hipStream_t stream, co
                            float* f, const int2* scat, const int4* tasks, long ncoef, const SliceMap& sm,
                            const float2* tws) {
     const dim3 grid((unsigned)(ntasks * batch));
-    if (LAYOUT == kSliced ? stream_sliced_coef(batch, ncoef) : batch >= kStreamCoefInMinBatch)
+    const bool past = LAYOUT == kSliced ? stream_sliced_coef(batch, ncoef)
+                      : LAYOUT == FCQT_INTERLEAVED ? batch >= kStreamCoefInMinBatch : stream_planes_in(batch, ncoef);
+    if (past)
         hipLaunchKernelGGL((k_scatter_bands<LAYOUT, Store::kPlain, true, true>), grid, dim3(kBandThreads), 0, stream,
                            cre, cim, f, scat, tasks, (int)batch, ncoef, sm, tws, (int)ntasks);
     else if (batch > kBandWriteThroughMaxBatch)

@@ -30,8 +30,15 @@ static_assert(kAnalysisChunk == 128 && kAnalysisChunkMinBatch == 256, "chunk con
 //   x:      B = 96 104.4 / 96.7, 127 140.8 / 133.3, but the analysis alone
 //           112 53.5 / 56.2, 120 58.2 / 59.3, 127 62.2 / 62.4, 160 80.1 / 75.0
 //   y:      B = 105 116.2 / 113.5, 127 140.8 / 137.8, 144 165.6 / 162.9 (with x)
-//   coefficients read by the scatter (with x, y): B = 127 130.5 / 138.9,
-//           136 147.9 / 149.6, 144 162.9 / 153.7, 160 189.5 / 166.8
+//   coefficient planes read by the scatter (with x, y): once an analysis's buffers
+//           (x, W, X, planes) hold 259 MB, a little more than the cache, which the planes do
+//           not outlive: 140 slices; 165 in the layout of 99,072 coefficients. B = 132
+//           146.2 / 144.5, 136 147.4 / 145.5, 144 159.5 / 155.0, 160 188.2 / 169.8; that layout 144 137.3 / 143.4,
+//           160 158.4 / 160.6, 164 162.0 / 161.1, 172 177.5 / 165.5 (the synthesis alone
+//           144 82.2 / 83.1, 164 93.7 / 93.9, 172 97.7 / 96.9; 144 76.3 / 77.5, 168 88.7 / 87.0)
+//   interleaved coefficients read: from 140 slices on in both layouts (training steps, which also
+//           read their gradients so, 140 389.0 / 378.9, 160 429.5 / 421.3; 353.8 / 346.6, 386.9 /
+//           382.2; round trips without gradients 140 149.9 / 148.8, 160 170.6 / 164.9; 133.4 / 133.5, 149.4 / 146.7)
 //   coefficients written by the route (with those): B = 160 166.8 / 167.2,
 //           176 183.9 / 182.8, 200 210.3 / 206.4, 512 592 / 550; the analysis
 //           alone 256 134.7 / 117.4, 512 271.8 / 221.2
@@ -56,6 +63,7 @@ static_assert(kAnalysisChunk == 128 && kAnalysisChunkMinBatch == 256, "chunk con
 // are not streamed.
 constexpr int64_t kStreamXMinBatch = 124;
 constexpr int64_t kStreamYMinBatch = 105;
+constexpr int64_t kStreamPlanesInBytes = 259000000;
 constexpr int64_t kStreamCoefInMinBatch = 140;
 constexpr int64_t kStreamCoefOutMinBatch = 192;
 constexpr int64_t kStreamNewCoefOutMinBatch = 140;
@@ -67,6 +75,9 @@ constexpr int64_t kStreamSlicedCoefBytes = 340000000;
 inline int64_t analysis_bytes(int64_t batch, int64_t ncoef) { return batch * (4 * FCQT_N + 16 * FCQT_L + 8 * ncoef); }
 inline int64_t round_trip_bytes(int64_t batch, int64_t ncoef) {
     return analysis_bytes(batch, ncoef) + batch * (8 * FCQT_FROW + 4 * FCQT_N);
+}
+inline bool stream_planes_in(int64_t batch, int64_t ncoef) {
+    return analysis_bytes(batch, ncoef) >= kStreamPlanesInBytes;
 }
 inline bool stream_sliced_coef(int64_t batch, int64_t ncoef) {
     return round_trip_bytes(batch, ncoef) >= kStreamSlicedCoefBytes;
