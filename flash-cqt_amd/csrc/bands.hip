@@ -98,7 +98,7 @@ static void launch_route(int64_t ntasks, int64_t batch, hipStream_t stream, cons
                   "batch ranges: plain task-major, write-through task-major, write-through slice-major, "
                   "plain slice-major");
     const bool past = LAYOUT == kSliced ? stream_sliced_coef(total, ncoef)
-                      : total >= (LAYOUT == FCQT_INTERLEAVED ? kStreamNewCoefOutMinBatch : kStreamCoefOutMinBatch);
+                      : LAYOUT == FCQT_INTERLEAVED ? total >= kStreamInterleavedMinBatch : stream_planes_out(total, ncoef);
     if (past)
         hipLaunchKernelGGL((k_route_bands<LAYOUT, Store::kStream, true>), grid, dim3(kBandThreads), 0, stream, xs, cre,
                            cim, rec, tasks, (int)batch, ncoef, sm, tws, (int)ntasks);
@@ -122,7 +122,7 @@ static void launch_scatter(int64_t ntasks, int64_t batch, hipStream_t stream, co
                            const float2* tws) {
     const dim3 grid((unsigned)(ntasks * batch));
     const bool past = LAYOUT == kSliced ? stream_sliced_coef(batch, ncoef)
-                      : LAYOUT == FCQT_INTERLEAVED ? batch >= kStreamCoefInMinBatch : stream_planes_in(batch, ncoef);
+                      : LAYOUT == FCQT_INTERLEAVED ? batch >= kStreamInterleavedMinBatch : stream_planes_in(batch, ncoef);
     if (past)
         hipLaunchKernelGGL((k_scatter_bands<LAYOUT, Store::kPlain, true, true>), grid, dim3(kBandThreads), 0, stream,
                            cre, cim, f, scat, tasks, (int)batch, ncoef, sm, tws, (int)ntasks);

@@ -22,51 +22,70 @@ static_assert(kAnalysisChunk == 128 && kAnalysisChunkMinBatch == 256, "chunk con
 
 // From these sizes on a buffer is written or read past the caches
 // (Store::kStream, load_in<true>). Per slice a round trip touches x, W, X,
-// the coefficients, F and y: 2.7 MB, so about 96 slices fill the 256 MB
-// memory-side cache, and past that a buffer without a nearby reader only
-// pushes W, X and F out to HBM. Measured as loops over three inputs, kept in
-// the caches against streamed (us, headline layout; round trip, or the
-// direction that is named):
-//   x:      B = 96 104.4 / 96.7, 127 140.8 / 133.3, but the analysis alone
-//           112 53.5 / 56.2, 120 58.2 / 59.3, 127 62.2 / 62.4, 160 80.1 / 75.0
-//   y:      B = 105 116.2 / 113.5, 127 140.8 / 137.8, 144 165.6 / 162.9 (with x)
-//   coefficient planes read by the scatter (with x, y): once an analysis's buffers
-//           (x, W, X, planes) hold 259 MB, a little more than the cache, which the planes do
-//           not outlive: 140 slices; 165 in the layout of 99,072 coefficients. B = 132
-//           146.2 / 144.5, 136 147.4 / 145.5, 144 159.5 / 155.0, 160 188.2 / 169.8; that layout 144 137.3 / 143.4,
-//           160 158.4 / 160.6, 164 162.0 / 161.1, 172 177.5 / 165.5 (the synthesis alone
-//           144 82.2 / 83.1, 164 93.7 / 93.9, 172 97.7 / 96.9; 144 76.3 / 77.5, 168 88.7 / 87.0)
-//   interleaved coefficients read: from 140 slices on in both layouts (training steps, which also
-//           read their gradients so, 140 389.0 / 378.9, 160 429.5 / 421.3; 353.8 / 346.6, 386.9 /
-//           382.2; round trips without gradients 140 149.9 / 148.8, 160 170.6 / 164.9; 133.4 / 133.5, 149.4 / 146.7)
-//   coefficients written by the route (with those): B = 160 166.8 / 167.2,
-//           176 183.9 / 182.8, 200 210.3 / 206.4, 512 592 / 550; the analysis
-//           alone 256 134.7 / 117.4, 512 271.8 / 221.2
-//   W read by the row pass (with those): B = 192 194.7 / 194.9,
-//           256 266.1 / 257.7, 512 550 / 518; not in the 128-slice chunks of
-//           fcqt_sliced_analysis, whose W is in the caches (256 slices 125.5 / 125.8,
-//           320 166.5 / 167.9, 512 263 / 263; layout (4, 3) x (12, 48) 109.1 / 110.5, 146.5 / 148.1, 231 / 229)
-// TrainableCQT's coefficients (interleaved) go to a new buffer each call, so
-// nothing in the caches is there for them: written past the caches from 140
-// slices on, training steps at 144 / 160 / 176 slices 404 / 436 / 469 -> 386 / 418 /
-// 460 us and round trips without gradients 153.5 / 167.7 / 183.1 -> 151.8 / 163.9 /
-// 177.7 (from 105 on steps gain as much, but round trips lose 4 us up to 127).
-// So do SlicedCQT's, and streaming both their ends pays earlier, from where a
-// round trip's buffers hold 340 MB (126 slices; 140 in the layout (4, 3) x (12, 48) of
-// 99,072 coefficients against 132,992): round trips at 105 / 112 / 120 / 128 / 136 /
-// 144 / 160 slices 120.5 / 125.1 / 132.7 / 142.6 / 162.0 / 181.3 / 205.3 kept, 126.7 /
-// 130.5 / 137.1 / 142.9 / 160.9 / 165.0 / 176.6 streamed; in that layout 108.2 / 112.5 /
-// 116.8 / 123.5 / 142.4 / 150.8 / 177.4 against 113.3 / 117.5 / 123.3 / 128.6 / 144.9 /
-// 148.9 / 163.8 (two signals of half as many slices alike). So does its output from kStreamYMinBatch on:
-// 120 slices 137.6 / 135.7, 160 184.3 / 178.3, 224 246.4 / 239.2, its inverse
-// alone at 512 304.4 / 292.1. Its signals are read twice (the overlap), so those
-// are not streamed.
+// the coefficients, F and y: 2.7 MB in the headline layout, so about 96 slices
+// fill the 256 MB memory-side cache, and past that a buffer without a nearby
+// reader only pushes W, X and F out to HBM. Limits that depend on the
+// coefficients' size are in bytes. Measured on one set of buffers over three
+// inputs in turn, kept in the caches / streamed, us; A the headline layout
+// (132,992 coefficients), B the layout (4, 3) x (12, 48) (99,072); rt a round
+// trip, fwd and bwd one direction alone:
+//
+//   x, 124 slices
+//     A rt   96 106.2 / 99.3   112 118.5 / 113.4   128 138.6 / 131.8   144 156.0 / 156.2
+//     A fwd  112 53.6 / 54.5   120 58.5 / 58.7     128 62.2 / 61.0     160 79.5 / 75.8
+//     B rt   96 91.6 / 89.5    112 104.9 / 102.2   128 120.4 / 114.6   160 159.4 / 160.0
+//     B fwd  112 47.4 / 48.5   120 50.0 / 52.0     128 52.8 / 54.4     136 59.7 / 59.2
+//     Inputs never seen before (24 in turn) are no slower streamed at any size from
+//     96 on (A fwd 112 54.6 / 54.2, B fwd 128 55.2 / 54.0); the losses above are of
+//     analyses that repeat an input which the cache still holds.
+//   y, 105 slices (its reader, if any, is the caller)
+//     A rt   105 116.0 / 112.6  120 132.2 / 128.1  136 150.9 / 150.8   200 203.6 / 200.1
+//     A bwd  105 65.1 / 63.9    120 70.8 / 70.6    144 83.9 / 83.9
+//     B rt   105 102.8 / 99.9   120 116.7 / 111.8  136 130.7 / 125.9   200 180.5 / 176.8
+//     B bwd  105 58.9 / 57.6    120 64.0 / 64.2    144 77.6 / 77.7
+//     training steps, whose loss reads y: A 105 304.8 / 305.2, 112 318.5 / 324.1,
+//     124 353.0 / 348.5, 136 387.0 / 394.0, 144 389.9 / 388.2; B 112 287.2 / 286.6,
+//     127 318.8 / 325.7, 136 347.8 / 354.4, 144 356.0 / 355.0 (-1.5 to +2%)
+//   coefficient planes read by the scatter, x + W + X + planes of 259 MB: the planes
+//   just written no longer outlive the rest of the analysis (A 140 slices, B 165)
+//     A rt   132 146.2 / 144.5  144 159.5 / 155.0  152 170.6 / 164.1   160 188.2 / 169.8
+//     A bwd  132 77.6 / 78.0    144 82.2 / 83.1    164 93.7 / 93.9     172 97.7 / 96.9
+//     B rt   144 137.3 / 143.4  160 158.4 / 160.6  164 162.0 / 161.1   172 177.5 / 165.5
+//     B bwd  144 76.3 / 77.5    164 83.9 / 85.1    168 88.7 / 87.0     172 88.4 / 87.6
+//   coefficient planes written by the route, the same buffers of 425 MB (A 230, B 270):
+//   the engine's planes are rewritten on every call, so the cache still holds a part
+//     A rt   200 204.3 / 206.3  216 217.1 / 217.6  240 256.6 / 239.3   272 312.4 / 271.2
+//     A fwd  200 90.5 / 94.8    216 99.0 / 100.0   240 110.7 / 109.1   280 148.9 / 124.4
+//     B rt   216 192.7 / 196.8  240 214.6 / 223.3  264 244.2 / 240.1   280 277.9 / 249.5
+//     B fwd  216 83.8 / 90.1    240 93.5 / 99.2    272 107.5 / 109.0   288 117.1 / 115.9
+//   TrainableCQT's coefficients (interleaved, a new buffer on each call, so that the
+//   cache holds nothing of it), 140 slices, written
+//     A step 136 402.3 / 387.7  144 407.2 / 393.5  160 433.0 / 428.5   192 504.3 / 493.1
+//     A rt   128 132.8 / 140.0  136 151.0 / 150.8  144 154.9 / 154.9   160 169.8 / 167.7
+//     B step 136 361.3 / 348.8  144 368.4 / 359.9  160 404.1 / 387.5   192 452.6 / 445.8
+//     B rt   128 114.9 / 123.2  136 128.6 / 132.5  144 139.7 / 138.5   160 150.5 / 148.7
+//   and read, with the gradients, which are read as coefficients too
+//     A step 132 385.4 / 368.0  140 389.0 / 378.9  160 429.5 / 421.3   172 453.3 / 450.2
+//     A rt   132 142.5 / 143.3  140 149.9 / 148.8  160 170.6 / 164.9   172 182.8 / 175.7
+//     B step 132 340.5 / 335.8  140 353.8 / 346.6  160 386.9 / 382.2   172 415.8 / 413.8
+//     B rt   132 121.1 / 123.9  140 133.4 / 133.5  160 149.4 / 146.7   172 162.0 / 157.7
+//   W read by the row pass, 192 slices of one launch (the chunks of
+//   fcqt_sliced_analysis stay below: their W was written just before)
+//     A rt   192 196.6 / 196.2  224 227.4 / 227.3  256 268.6 / 262.8   320 333.6 / 319.6
+//     B rt   192 183.8 / 183.6  224 205.1 / 204.0  256 235.8 / 233.4   320 299.7 / 286.3
+//   SlicedCQT's coefficients (a new buffer on each call, both ends), a round trip's
+//   buffers of 340 MB (A 126 slices, B 140)
+//     A rt   105 120.5 / 126.7  120 132.7 / 137.1  128 143.4 / 139.9   144 181.3 / 165.0
+//     A fwd  105 54.1 / 56.8    120 60.1 / 62.2    126 64.4 / 61.7     144 80.4 / 76.1
+//     B rt   105 108.2 / 113.3  120 116.8 / 123.3  136 143.6 / 141.6   160 177.4 / 163.8
+//     B fwd  120 51.9 / 53.7    136 64.0 / 64.0    140 63.4 / 65.2     144 71.2 / 66.8
+//   SlicedCQT's output, kStreamYMinBatch: rt 120 137.6 / 135.7, 160 184.3 / 178.3, 224 246.4 /
+//   239.2, bwd 512 304.4 / 292.1. Its signals are read twice (the overlap) and not streamed.
 constexpr int64_t kStreamXMinBatch = 124;
 constexpr int64_t kStreamYMinBatch = 105;
 constexpr int64_t kStreamPlanesInBytes = 259000000;
-constexpr int64_t kStreamCoefInMinBatch = 140;
-constexpr int64_t kStreamCoefOutMinBatch = 192;
-constexpr int64_t kStreamNewCoefOutMinBatch = 140;
+constexpr int64_t kStreamPlanesOutBytes = 425000000;
+constexpr int64_t kStreamInterleavedMinBatch = 140;
 constexpr int64_t kStreamWMinBatch = 192;
 constexpr int64_t kStreamSlicedCoefBytes = 340000000;
 
@@ -78,6 +97,9 @@ inline int64_t round_trip_bytes(int64_t batch, int64_t ncoef) {
 }
 inline bool stream_planes_in(int64_t batch, int64_t ncoef) {
     return analysis_bytes(batch, ncoef) >= kStreamPlanesInBytes;
+}
+inline bool stream_planes_out(int64_t batch, int64_t ncoef) {
+    return analysis_bytes(batch, ncoef) >= kStreamPlanesOutBytes;
 }
 inline bool stream_sliced_coef(int64_t batch, int64_t ncoef) {
     return round_trip_bytes(batch, ncoef) >= kStreamSlicedCoefBytes;
