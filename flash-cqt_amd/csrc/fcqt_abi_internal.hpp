@@ -52,12 +52,14 @@ static_assert(kAnalysisChunk == 128 && kAnalysisChunkMinBatch == 256, "chunk con
 //     A bwd  132 77.6 / 78.0    144 82.2 / 83.1    164 93.7 / 93.9     172 97.7 / 96.9
 //     B rt   144 137.3 / 143.4  160 158.4 / 160.6  164 162.0 / 161.1   172 177.5 / 165.5
 //     B bwd  144 76.3 / 77.5    164 83.9 / 85.1    168 88.7 / 87.0     172 88.4 / 87.6
-//   coefficient planes written by the route, the same buffers of 425 MB (A 230, B 270):
-//   the engine's planes are rewritten on every call, so the cache still holds a part
-//     A rt   200 204.3 / 206.3  216 217.1 / 217.6  240 256.6 / 239.3   272 312.4 / 271.2
-//     A fwd  200 90.5 / 94.8    216 99.0 / 100.0   240 110.7 / 109.1   280 148.9 / 124.4
-//     B rt   216 192.7 / 196.8  240 214.6 / 223.3  264 244.2 / 240.1   280 277.9 / 249.5
-//     B fwd  216 83.8 / 90.1    240 93.5 / 99.2    272 107.5 / 109.0   288 117.1 / 115.9
+//   coefficient planes written by the route, the same buffers of 354 MB (A and C 192, B 224):
+//   round trips gain from about there on; analyses alone rewrite planes of which the
+//   cache still holds a part and gain later (C the layout (2, 5, 2) x (4, 8, 64), 131,968)
+//     A rt   192 197.7 / 197.7  216 217.1 / 217.6  229 246.4 / 234.8   272 312.4 / 271.2
+//     A fwd  192 88.7 / 89.2    216 99.0 / 100.0   229 107.7 / 108.0   280 148.9 / 124.4
+//     C rt   200 211.7 / 202.6  229 239.0 / 228.0      C fwd 200 92.5 / 92.0   229 107.5 / 104.1
+//     B rt   200 182.4 / 185.4  216 192.7 / 196.8  229 207.4 / 207.5   260 247.6 / 238.9
+//     B fwd  200 80.3 / 84.5    216 83.8 / 90.1    229 91.0 / 93.9     280 111.5 / 111.7
 //   TrainableCQT's coefficients (interleaved, a new buffer on each call, so that the
 //   cache holds nothing of it), 140 slices, written
 //     A step 136 402.3 / 387.7  144 407.2 / 393.5  160 433.0 / 428.5   192 504.3 / 493.1
@@ -84,7 +86,7 @@ static_assert(kAnalysisChunk == 128 && kAnalysisChunkMinBatch == 256, "chunk con
 constexpr int64_t kStreamXMinBatch = 124;
 constexpr int64_t kStreamYMinBatch = 105;
 constexpr int64_t kStreamPlanesInBytes = 259000000;
-constexpr int64_t kStreamPlanesOutBytes = 425000000;
+constexpr int64_t kStreamPlanesOutBytes = 353600000;
 constexpr int64_t kStreamInterleavedMinBatch = 140;
 constexpr int64_t kStreamWMinBatch = 192;
 constexpr int64_t kStreamSlicedCoefBytes = 340000000;

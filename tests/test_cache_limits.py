@@ -26,6 +26,6 @@ def _first(tmp_path, rule):
 
 @pytest.mark.parametrize("rule,first", [("stream_sliced_coef(batch, ncoef)", (126, 140)),
                                         ("stream_planes_in(batch, ncoef)", (140, 165)),
-                                        ("stream_planes_out(batch, ncoef)", (230, 270))])
+                                        ("stream_planes_out(batch, ncoef)", (192, 224))])
 def test_first_batch_past_the_caches(tmp_path, rule, first):
     assert _first(tmp_path, rule) == first
