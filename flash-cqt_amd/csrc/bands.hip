@@ -243,7 +243,7 @@ extern "C" int fcqt_sliced_analysis(const fcqt_tables* tab, const int32_t* route
         const int64_t na = nsig - a < ns ? nsig - a : ns;
         for (int64_t c = 0; c < nslices; c += cs) {
             const int64_t nc = nslices - c < cs ? nslices - c : cs;
-            if (int e = fcqt_slice_fft_fwd(tab, sig + a * sig_len, sig_len, window, na, nc, c, 0, xs, work, stream))
+            if (int e = slice_fft_fwd(tab, sig + a * sig_len, sig_len, window, na, nc, c, 0, xs, work, batch, stream))
                 return e;
             launch_route<kSliced>(tab->ntasks, na * nc, stream, reinterpret_cast<const float2*>(xs), coef, coef,
                                   reinterpret_cast<const int2*>(route), reinterpret_cast<const int4*>(tab->tasks),

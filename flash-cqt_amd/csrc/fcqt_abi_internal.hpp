@@ -71,8 +71,9 @@ static_assert(kAnalysisChunk == 128 && kAnalysisChunkMinBatch == 256, "chunk con
 //     A rt   132 142.5 / 143.3  140 149.9 / 148.8  160 170.6 / 164.9   172 182.8 / 175.7
 //     B step 132 340.5 / 335.8  140 353.8 / 346.6  160 386.9 / 382.2   172 415.8 / 413.8
 //     B rt   132 121.1 / 123.9  140 133.4 / 133.5  160 149.4 / 146.7   172 162.0 / 157.7
-//   W read by the row pass, 192 slices of one launch (the chunks of
-//   fcqt_sliced_analysis stay below: their W was written just before)
+//   W read by the row pass, 192 slices of a whole call (in the 128-slice chunks of
+//   fcqt_sliced_analysis, whose W was written just before, either form is within 1%:
+//   A fwd 384 188.9 / 190.7, 512 263.9 / 262.2, rt 320 364.0 / 360.3, 512 566.0 / 567.4)
 //     A rt   192 196.6 / 196.2  224 227.4 / 227.3  256 268.6 / 262.8   320 333.6 / 319.6
 //     B rt   192 183.8 / 183.6  224 205.1 / 204.0  256 235.8 / 233.4   320 299.7 / 286.3
 //   SlicedCQT's coefficients (a new buffer on each call, both ends), a round trip's
@@ -120,6 +121,12 @@ int check_band_args(const fcqt_tables* tab, const int32_t* rec, const float* cre
 // in packed_fft.hip.
 int packed_fft_inv(const fcqt_tables* tab, const int32_t* ovf, const float* f, float* y, float* work, int64_t batch,
                    bool last, hipStream_t stream);
+
+// fcqt_slice_fft_fwd of one chunk of a call of `total` slices (which sets
+// the cache choices); defined in packed_fft.hip.
+int slice_fft_fwd(const fcqt_tables* tab, const float* sig, int64_t sig_len, const float* window, int64_t nsig,
+                  int64_t nslices, int64_t first, int64_t origin, float* xs, float* work, int64_t total,
+                  hipStream_t stream);
 
 // The inverse passes of one streamed slice per signal with the half-slice
 // overlap-add in the row pass's store (arguments checked by the caller);

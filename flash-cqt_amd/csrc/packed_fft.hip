@@ -91,15 +91,16 @@ static int launch_fwd_passes(const float2* x, float2* work, float2* xs, const fl
     return launch_status();
 }
 
-// Sliced framing reads every sample twice, so its signals are not streamed.
+// total: slices of the whole call that this batch is a chunk of.
 static int fwd_passes(const float2* x, float2* work, float2* xs, const float2* twp, const float2* twh,
-                      const float2* tws, const SliceSrc& src, bool sliced, int64_t batch, hipStream_t stream) {
+                      const float2* tws, const SliceSrc& src, bool sliced, int64_t batch, int64_t total,
+                      hipStream_t stream) {
     if (batch <= kNarrowMaxBatch)
         return launch_fwd_passes<kColsNarrow, kRowsNarrow>(x, work, xs, twp, twh, tws, src, sliced, batch, stream);
-    if (batch >= kStreamWMinBatch)
+    if (total >= kStreamWMinBatch)
         return launch_fwd_passes<kColsWide, kRowsWide, true, true>(x, work, xs, twp, twh, tws, src, sliced, batch,
                                                                    stream);
-    if (batch >= kStreamXMinBatch)
+    if (total >= kStreamXMinBatch)
         return launch_fwd_passes<kColsWide, kRowsWide, true>(x, work, xs, twp, twh, tws, src, sliced, batch, stream);
     return launch_fwd_passes<kColsWide, kRowsWide>(x, work, xs, twp, twh, tws, src, sliced, batch, stream);
 }
@@ -262,7 +263,7 @@ extern "C" int fcqt_packed_fft_fwd(const fcqt_tables* tab, const float* x, float
     return fwd_passes(reinterpret_cast<const float2*>(x), reinterpret_cast<float2*>(work),
                       reinterpret_cast<float2*>(xs), reinterpret_cast<const float2*>(tab->tw_pass),
                       reinterpret_cast<const float2*>(tab->tw_half), reinterpret_cast<const float2*>(tab->tw_stage),
-                      SliceSrc{nullptr, nullptr, 1, 1, 0, 0, 0, nullptr, 1, 1, 1}, false, batch, stream);
+                      SliceSrc{nullptr, nullptr, 1, 1, 0, 0, 0, nullptr, 1, 1, 1}, false, batch, batch, stream);
 }
 
 int fcqt::packed_fft_inv(const fcqt_tables* tab, const int32_t* ovf, const float* f, float* y, float* work,
@@ -283,9 +284,9 @@ extern "C" int fcqt_packed_fft_inv(const fcqt_tables* tab, const int32_t* ovf, c
     return packed_fft_inv(tab, ovf, f, y, work, batch, false, stream);
 }
 
-extern "C" int fcqt_slice_fft_fwd(const fcqt_tables* tab, const float* sig, int64_t sig_len, const float* window,
-                                  int64_t nsig, int64_t nslices, int64_t first, int64_t origin, float* xs,
-                                  float* work, hipStream_t stream) {
+int fcqt::slice_fft_fwd(const fcqt_tables* tab, const float* sig, int64_t sig_len, const float* window, int64_t nsig,
+                        int64_t nslices, int64_t first, int64_t origin, float* xs, float* work, int64_t total,
+                        hipStream_t stream) {
     if (!tab || !sig || !window || !xs || !work || sig_len < 1 || nsig < 1 || nslices < 1) return FCQT_EARG;
     if (first < 0 || first > kMaxBatch || origin < -(int64_t)kN || origin > (int64_t)kN * kMaxBatch)
         return FCQT_EARG;
@@ -302,7 +303,13 @@ extern "C" int fcqt_slice_fft_fwd(const fcqt_tables* tab, const float* sig, int6
                       reinterpret_cast<const float2*>(tab->tw_stage),
                       SliceSrc{sig, window, (long)sig_len, (int)nslices, (long)first, (long)origin, pairs, nullptr,
                                (long)sig_len, (long)sig_len, (long)sig_len},
-                      true, batch, stream);
+                      true, batch, total, stream);
+}
+
+extern "C" int fcqt_slice_fft_fwd(const fcqt_tables* tab, const float* sig, int64_t sig_len, const float* window,
+                                  int64_t nsig, int64_t nslices, int64_t first, int64_t origin, float* xs,
+                                  float* work, hipStream_t stream) {
+    return slice_fft_fwd(tab, sig, sig_len, window, nsig, nslices, first, origin, xs, work, nsig * nslices, stream);
 }
 
 extern "C" int fcqt_stream_analysis(const fcqt_tables* tab, const int32_t* route, const int32_t* groups,
@@ -331,7 +338,7 @@ extern "C" int fcqt_stream_analysis(const fcqt_tables* tab, const int32_t* route
                            reinterpret_cast<const float2*>(tab->tw_stage),
                            SliceSrc{prev, window, 2 * kHop, 1, (long)slice, kHop * ((long)slice - 1), pairs, next,
                                     (long)prev_stride, (long)next_stride, kHop},
-                           true, nsig, stream))
+                           true, nsig, nsig, stream))
         return e;
     return fcqt_route_bands_sliced(tab, route, groups, xs, coef, nsig, 1, slice, stream);
 }
