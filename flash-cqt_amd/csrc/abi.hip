@@ -21,7 +21,7 @@ __global__ __launch_bounds__(256) void k_fill_zero(float4* __restrict__ p4, long
 // (1.3 MB) in one launch instead of three copies by the runtime, the whole call
 // 54.1 -> 43.9 us (torch's foreach copy, 64 Ki elements per workgroup, was slower
 // than the three copies).
-constexpr int64_t kCopyPerWg = 8192;
+constexpr int64_t kCopyPerWg = FCQT_COPY_SHARE;
 struct CopyArgs {
     const char* src[FCQT_COPY_MAX];
     char* dst[FCQT_COPY_MAX];
@@ -99,7 +99,7 @@ extern "C" int fcqt_copy_buffers(const void* const* src, void* const* dst, const
         a.bytes[i] = (long)bytes[i];
         a.first[i] = (unsigned)wgs;
         wgs += (bytes[i] + kCopyPerWg - 1) / kCopyPerWg;
-        if (wgs > 1 << 23) return FCQT_EARG;         // 64 GiB in all: the grid's limit
+        if (wgs > FCQT_COPY_BYTES / kCopyPerWg) return FCQT_EARG;
     }
     a.first[count] = (unsigned)wgs;
     a.count = count;

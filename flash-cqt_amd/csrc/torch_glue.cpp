@@ -285,16 +285,21 @@ py::object guarded(F f, const A&... a) {
 }
 
 // Copies of the tensors (t.clone() each) with one launch of fcqt_copy_buffers, or
-// None where one of them is not a plain dense tensor of the current GPU.
+// None where one of them is not a plain dense tensor of the current GPU or they
+// pass that launch's 64 GiB.
 py::object clones(const std::vector<Tensor>& ts, int64_t copy_fn) {
     if (ts.empty() || ts.size() > FCQT_COPY_MAX || !plain_call()) return py::none();
     const c10::Device device(c10::kCUDA, c10::hip::current_device());
     const void* src[FCQT_COPY_MAX];
     void* dst[FCQT_COPY_MAX];
     int64_t bytes[FCQT_COPY_MAX];
-    for (const Tensor& t : ts)
+    size_t total = 0;
+    for (const Tensor& t : ts) {
         if (!plain_tensor(device, t, t.scalar_type()) || !t.is_non_overlapping_and_dense() || t.numel() == 0)
             return py::none();
+        total += t.nbytes() + FCQT_COPY_SHARE;         // a buffer's last workgroup may be short
+    }
+    if (total > FCQT_COPY_BYTES) return py::none();
     std::vector<Tensor> out;
     for (size_t i = 0; i < ts.size(); ++i) {
         out.push_back(at::empty_like(ts[i]));

@@ -451,10 +451,13 @@ int fcqt_stream_synthesis(const fcqt_tables* tab, const int32_t* scat, const int
 int fcqt_fill_zero(float* buf, int64_t n, hipStream_t stream);
 
 /* Copy bytes[i] bytes (>= 1) from src[i] to dst[i] for i < count <=
- * FCQT_COPY_MAX with one kernel: the outputs of a replayed graph into buffers of
- * their own. The three arrays are host memory, read before the call returns; the
+ * FCQT_COPY_MAX with one kernel, at most FCQT_COPY_BYTES in all (each buffer rounded
+ * up to FCQT_COPY_SHARE, a workgroup's share): the outputs of a replayed graph
+ * into buffers of their own. The three arrays are host memory, read before the call returns; the
  * buffers are device memory of any alignment and do not overlap. */
 #define FCQT_COPY_MAX 16
+#define FCQT_COPY_SHARE 8192
+#define FCQT_COPY_BYTES 68719476736    /* 64 GiB: 2^23 workgroups, the grid's limit */
 int fcqt_copy_buffers(const void* const* src, void* const* dst, const int64_t* bytes, int count, hipStream_t stream);
 
 #ifdef __cplusplus

@@ -56,3 +56,26 @@ def test_graphed_outputs_are_copies_of_every_kind():
     simple = Graphed(lambda a: (a + 1, [a.t() * 2]), x)       # every output plain: one launch
     for s in (1.0, 2.0, 3.0):
         assert same(simple(x * s), (x * s + 1, [(x * s).t() * 2]))
+
+
+def test_outputs_past_one_launch_are_cloned_one_by_one():
+    """More than the copy kernel takes in one launch (here one 5 GiB tensor 13
+    times, 65 GiB) is declined before anything is allocated for it; Graphed then
+    clones each output."""
+    import ctypes as c
+    from flash_cqt import _native
+    fn = c.cast(_native.load().fcqt_copy_buffers, c.c_void_p).value
+    big = torch.empty(5 << 30, dtype=torch.uint8, device="cuda")
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    assert _native.load_glue().clones([big] * 13, fn) is None
+    assert torch.cuda.max_memory_allocated() == before
+    del big
+    torch.cuda.empty_cache()
+
+
+def test_copy_buffers_refuses_more_than_one_launch_takes():
+    from flash_cqt import _native
+    lib, p = _native.load(), (ctypes.c_void_p * 2)(4096, 4096)
+    for sizes in ((1 << 36, 1), ((1 << 36) - 8192, 8193)):
+        assert lib.fcqt_copy_buffers(p, p, (ctypes.c_int64 * 2)(*sizes), 2, None) == 1
