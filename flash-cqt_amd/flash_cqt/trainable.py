@@ -35,13 +35,25 @@ class TrainableCQT:
         self._glue = self.f.attach_glue()
 
     def _plain(self, tensors):
-        """The host glue when every tensor is an ordinary one and the engine
-        runs the library it was attached to (the glue itself declines what
-        else it does not take), else None."""
-        if self._glue is not None and self.f.lib is self._lib and not torch.compiler.is_compiling() \
-                and all(type(t) is torch.Tensor or type(t) is torch.nn.Parameter for t in tensors):
-            return self._glue
+        """The host glue when every tensor is an ordinary one, the engine is the
+        one that the glue belongs to with the library it was attached to, and
+        the directions below are this class's own (the glue itself declines
+        what else it does not take), else None."""
+        glue, f = self._glue, self.f
+        if glue is not None and f._glue is glue and f.lib is self._lib and not torch.compiler.is_compiling() \
+                and all(type(t) is torch.Tensor or type(t) is torch.nn.Parameter for t in tensors) \
+                and self._own_directions():
+            return glue
         return None
+
+    def _own_directions(self):
+        """No direction replaced, by a subclass, on the class or on this object:
+        the glue would pass such a method by."""
+        cls = type(self)
+        for name, own in _DIRECTIONS:
+            if getattr(cls, name) is not own:
+                return False
+        return self.__dict__.keys().isdisjoint(_NAMES)
 
     # ------------------------------------------------ engine directions
     # The inputs reaching these are [B, N] float32 or [B, ncoef] complex64,
@@ -162,6 +174,12 @@ class TrainableCQT:
         if flat.device != self.dev:
             raise ValueError(f"blocks are on {flat.device}, engine on {self.dev}")
         return _Synthesis.apply(flat.resolve_conj().contiguous(), self).reshape(*lead, N)
+
+
+# the methods that the host glue stands in for
+_NAMES = ("_launch_analysis", "_launch_synthesis", "_analysis", "_synthesis", "_adj_analysis", "_adj_synthesis",
+          "_base_of")
+_DIRECTIONS = tuple((n, getattr(TrainableCQT, n)) for n in _NAMES)
 
 
 class _Analysis(torch.autograd.Function):

@@ -75,3 +75,36 @@ def test_leaf_views_are_not_the_buffer(engine, base_grad):
     assert engine._base_of(parts, 6) is None
     with torch.no_grad():
         assert engine._base_of(parts, 6) is kc
+
+
+def test_replaced_directions_and_engines_are_not_passed_by(monkeypatch):
+    """The C++ path serves the class's own directions on the engine that it was
+    attached to, nothing else."""
+    import types
+    from flash_cqt.trainable import TrainableCQT
+    glue, lib = object(), object()
+
+    def make(cls):
+        t = cls.__new__(cls)
+        t.f, t._lib, t._glue = types.SimpleNamespace(lib=lib, _glue=glue), lib, glue
+        return t
+
+    class Same(TrainableCQT):
+        extra = 1
+
+    class Other(TrainableCQT):
+        def _synthesis(self, kc):
+            return super()._synthesis(kc) * 2
+    x = (torch.zeros(1),)
+    assert make(TrainableCQT)._plain(x) is glue and make(Same)._plain(x) is glue
+    assert make(Other)._plain(x) is None
+    t = make(TrainableCQT)
+    t._analysis = lambda v: v
+    assert t._plain(x) is None
+    t = make(TrainableCQT)
+    t.f = types.SimpleNamespace(lib=lib, _glue=None)               # another engine on the same library
+    assert t._plain(x) is None
+    t.f = types.SimpleNamespace(lib=lib, _glue=object())
+    assert t._plain(x) is None
+    monkeypatch.setattr(TrainableCQT, "_adj_analysis", lambda self, g: g)
+    assert make(TrainableCQT)._plain(x) is None
