@@ -149,13 +149,16 @@ def _open(path):
         "fcqt_persist_tune": ([ctypes.c_int, ctypes.c_int, ctypes.c_int, I64], ctypes.c_int),
         "fcqt_persist_trace": ([P, I64], ctypes.c_int),
     }
-    for name, (args, res) in sig.items():
-        fn = getattr(lib, name)
-        fn.argtypes = args
-        fn.restype = res
-    ver = lib.fcqt_abi_version()
+    # the version first: a library of another version may lack the rest
+    ver = lib.fcqt_abi_version() if hasattr(lib, "fcqt_abi_version") else None
     if ver != ABI_VERSION:
         raise NativeError(f"libflashcqt ABI {ver}, expected {ABI_VERSION}; rebuild")
+    for name, (args, res) in sig.items():
+        fn = getattr(lib, name, None)
+        if fn is None:
+            raise NativeError(f"{path} lacks {name}; rebuild")
+        fn.argtypes = args
+        fn.restype = res
     return lib
 
 

@@ -66,6 +66,21 @@ def test_abi_version(lib):
     assert lib.fcqt_abi_version() == _native.ABI_VERSION == 13
 
 
+def test_stale_libraries_are_refused_by_name_and_version(tmp_path):
+    """A library of the version before, or of this one without a function that
+    it declares, raises NativeError, not the loader's AttributeError."""
+    import shutil
+    import subprocess
+    from flash_cqt import _native
+    for version, text in ((_native.ABI_VERSION - 1, "ABI"), (_native.ABI_VERSION, "lacks"), (None, "ABI None")):
+        name = "fcqt_abi_version" if version else "other"
+        src, out = tmp_path / "stale.c", tmp_path / f"stale{version}.so"
+        src.write_text(f"int {name}(void) {{ return {version or 0}; }}\n")
+        subprocess.run([shutil.which("gcc") or "gcc", "-shared", "-fPIC", str(src), "-o", str(out)], check=True, timeout=60)
+        with pytest.raises(_native.NativeError, match=text):
+            _native._open(out)
+
+
 def test_header_constants_match_tables_and_kernels():
     """The layout macros of flashcqt.h, the device constants of fcqt_fft.hpp
     and the table builder's constants are one set of numbers."""
