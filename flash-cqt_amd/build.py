@@ -80,7 +80,8 @@ def glue_command(out=GLUE):
     inc = [base / "include", base / "include" / "torch" / "csrc" / "api" / "include",
            sysconfig.get_paths()["include"], "/opt/rocm/include"]
     return [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__",
-            "-DUSE_ROCM", "-DTORCH_EXTENSION_NAME=_fcqt_torch", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+            "-DUSE_ROCM", "-DTORCH_EXTENSION_NAME=_fcqt_torch", f'-DFCQT_TORCH_VERSION="{torch.__version__}"',
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
             *[a for d in inc for a in ("-isystem", str(d))], str(GLUE_SOURCE), "-o", str(out), f"-L{base / 'lib'}",
             "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python", "-lc10", "-lc10_hip"]
 
@@ -128,6 +129,7 @@ def build(verbose=False):
         print(text)
     if glue.returncode != 0:
         failed.append(f"host glue: compiler failed ({glue.returncode})")
+        GLUE.unlink(missing_ok=True)       # not the one of an earlier build beside a new library
     else:
         os.replace(glue_tmp, GLUE)
     if failed:

@@ -318,8 +318,11 @@ const void* address(int64_t p) { return reinterpret_cast<const void*>(p); }
 }  // namespace
 
 PYBIND11_MODULE(_fcqt_torch, m) {
-    // [t.as_strided(size, stride, offset) for size, stride, offset in args]
+    // what the loader compares with the library and the running torch
+    m.attr("abi_version") = FCQT_ABI_VERSION;
+    m.attr("torch_version") = FCQT_TORCH_VERSION;
     m.def("clones", [](const std::vector<Tensor>& ts, int64_t copy_fn) { return guarded(clones, ts, copy_fn); });
+    // [t.as_strided(size, stride, offset) for size, stride, offset in args]
     m.def("strided_views", [](const Tensor& t, const std::vector<std::tuple<std::vector<int64_t>, std::vector<int64_t>,
                                                                             int64_t>>& args) {
         std::vector<Tensor> out;

@@ -98,14 +98,24 @@ _glue = None
 
 
 def load_glue():
-    """The host glue module (csrc/torch_glue.cpp) that TrainableCQT and
-    SlicedCQT call where one C++ call replaces many small Python ones, or None
-    when it was not built: the Python paths then do the same work."""
+    """The host glue module (csrc/torch_glue.cpp) that TrainableCQT,
+    SlicedCQT and Graphed call where one C++ call replaces many small Python ones, or None
+    when it was not built: the Python paths then do the same work. It calls
+    the library's functions by address and torch's by its headers, so one built
+    for another ABI version or another torch raises NativeError."""
     global _glue
     if _glue is None and GLUE_PATH.exists():
-        spec = importlib.util.spec_from_file_location("_fcqt_torch", GLUE_PATH)
-        _glue = importlib.util.module_from_spec(spec)
-        spec.loader.exec_module(_glue)
+        try:
+            spec = importlib.util.spec_from_file_location("_fcqt_torch", GLUE_PATH)
+            mod = importlib.util.module_from_spec(spec)
+            spec.loader.exec_module(mod)
+        except ImportError as e:
+            raise NativeError(f"cannot load {GLUE_PATH}: {e}; rebuild") from e
+        built = (getattr(mod, "abi_version", None), getattr(mod, "torch_version", None))
+        if built != (ABI_VERSION, str(torch.__version__)):
+            raise NativeError(f"{GLUE_PATH} was built for ABI {built[0]} and torch {built[1]}, expected {ABI_VERSION} "
+                              f"and {torch.__version__}; rebuild")
+        _glue = mod
     return _glue
 
 

@@ -108,3 +108,44 @@ def test_replaced_directions_and_engines_are_not_passed_by(monkeypatch):
     assert t._plain(x) is None
     monkeypatch.setattr(TrainableCQT, "_adj_analysis", lambda self, g: g)
     assert make(TrainableCQT)._plain(x) is None
+
+
+def test_glue_of_another_build_is_refused(monkeypatch, tmp_path):
+    from flash_cqt import _native
+    mod = _native.load_glue()
+    assert mod is not None and (mod.abi_version, mod.torch_version) == (_native.ABI_VERSION, str(torch.__version__))
+    monkeypatch.setattr(_native, "_glue", None)
+    with monkeypatch.context() as m:
+        m.setattr(_native, "ABI_VERSION", _native.ABI_VERSION + 1)
+        with pytest.raises(_native.NativeError, match="rebuild"):
+            _native.load_glue()
+    with monkeypatch.context() as m:
+        m.setattr(torch, "__version__", "0.0.0")
+        with pytest.raises(_native.NativeError, match="torch"):
+            _native.load_glue()
+    broken = tmp_path / "_fcqt_torch.so"
+    broken.write_bytes(b"not a library")
+    monkeypatch.setattr(_native, "GLUE_PATH", broken)
+    with pytest.raises(_native.NativeError, match="rebuild"):
+        _native.load_glue()
+    monkeypatch.setattr(_native, "GLUE_PATH", tmp_path / "absent.so")
+    assert _native.load_glue() is None
+
+
+def test_failed_glue_build_leaves_none_behind(monkeypatch, tmp_path):
+    """build() with a host compiler that fails removes an earlier build's glue."""
+    import importlib.util
+    import pathlib
+    root = pathlib.Path(__file__).resolve().parents[1]
+    spec = importlib.util.spec_from_file_location("flashcqt_build_test", root / "flash-cqt_amd" / "build.py")
+    b = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(b)
+    old = tmp_path / "_fcqt_torch.so"
+    old.write_bytes(b"old")
+    monkeypatch.setattr(b, "GLUE", old)
+    monkeypatch.setattr(b, "OUT", tmp_path / "libflashcqt.so")
+    monkeypatch.setattr(b, "VARIANTS", {})
+    monkeypatch.setattr(b, "glue_command", lambda out: ["false"])
+    with pytest.raises(RuntimeError, match="glue"):
+        b.build()
+    assert not old.exists()
