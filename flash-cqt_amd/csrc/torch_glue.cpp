@@ -47,7 +47,9 @@ struct Engine : torch::CustomClassHolder {
     // the engine's current buffer set (leading rows serve any smaller batch);
     // Python publishes every change, so nothing here outlives a replaced set
     std::mutex mu;
-    std::mutex launching;     // a direction's launches stay together: they share the set
+    // a direction's launches stay together: they share the set (Python holds it too,
+    // as a context manager, around the launches of the calls that fwd and bwd decline)
+    std::mutex launching;
     int64_t rows = 0;
     Tensor X, W, F, FA;
     std::atomic<bool> captured{false};
@@ -369,6 +371,9 @@ PYBIND11_MODULE(_fcqt_torch, m) {
                  e->X = e->W = e->F = e->FA = Tensor();
                  e->captured = false;
              })
+        // waiting without the GIL: the holder may need it to get on
+        .def("__enter__", [](const Ref& e) { e->launching.lock(); }, py::call_guard<py::gil_scoped_release>())
+        .def("__exit__", [](const Ref& e, const py::args&) { e->launching.unlock(); })
         .def_property_readonly("captured", [](const Ref& e) { return e->captured.load(); })
         .def("fwd", [](const Ref& e, const Tensor& x) { return guarded(fwd, e, x); })
         .def("bwd", [](const Ref& e, const std::vector<Tensor>& parts) { return guarded(bwd, e, parts); });

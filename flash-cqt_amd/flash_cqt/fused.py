@@ -19,6 +19,7 @@ every result is bitwise reproducible.
 Table semantics follow fused.py:303-476; see flash_cqt/tables.py.
 """
 import ctypes
+import threading
 
 import numpy as np
 import torch
@@ -123,6 +124,10 @@ class FusedOctCQT:
         self._ws = {}          # batch size -> views of the set's leading rows
         self._wp = {}          # batch size -> their raw pointers
         self._glue = None      # the C++ host glue that uses the current set too
+        # held around a direction's launches by TrainableCQT, whose results are
+        # the caller's own, so that threads may share it on one stream (fwd and
+        # bwd here return views of the set, which the next call overwrites)
+        self._launching = threading.Lock()
 
     # ------------------------------------------------------------ buffers
 
@@ -214,6 +219,7 @@ class FusedOctCQT:
                                  up.ovf_scat, up.ovf_scat_a], t.ntasks, t.ncoef, t.coef_span,
                                 fn(self.lib.fcqt_analysis), fn(self.lib.fcqt_synthesis), self._table_mem,
                                 [list(g) for g in self.gspec], len(self.cqt.groups))
+        self._launching = self._glue           # its mutex: the C++ calls hold it too
         self._publish()
         return self._glue
 

@@ -70,9 +70,11 @@ class TrainableCQT:
         f._workspace(B)
         p = f._wp[B]
         kc = torch.empty(B, self.ncoef, dtype=torch.complex64, device=self.dev)
-        _native.check(f.lib.fcqt_analysis(f._ct, f._tp[table], x.data_ptr(), kc.data_ptr(), None,
-                                          _native.INTERLEAVED, p["X"], p["W"], B,
-                                          _native.stream_handle(self.dev.index)), "analysis")
+        stream = _native.stream_handle(self.dev.index)
+        with f._launching:
+            status = f.lib.fcqt_analysis(f._ct, f._tp[table], x.data_ptr(), kc.data_ptr(), None,
+                                         _native.INTERLEAVED, p["X"], p["W"], B, stream)
+        _native.check(status, "analysis")
         return kc
 
     def _launch_synthesis(self, kc, table, fbuf):
@@ -81,9 +83,11 @@ class TrainableCQT:
         f._fbuf(table, B)                  # the table's scatter buffer (FA on first adjoint use)
         p = f._wp[B]
         y = torch.empty(B, N, dtype=torch.float32, device=self.dev)
-        _native.check(f.lib.fcqt_synthesis(f._ct, f._tp[table], f._tp["ovf_" + table], kc.data_ptr(), None,
-                                           _native.INTERLEAVED, p[fbuf], p["W"], y.data_ptr(), B,
-                                           _native.stream_handle(self.dev.index)), "synthesis")
+        stream = _native.stream_handle(self.dev.index)
+        with f._launching:
+            status = f.lib.fcqt_synthesis(f._ct, f._tp[table], f._tp["ovf_" + table], kc.data_ptr(), None,
+                                          _native.INTERLEAVED, p[fbuf], p["W"], y.data_ptr(), B, stream)
+        _native.check(status, "synthesis")
         return y
 
     def _analysis(self, x):

@@ -208,3 +208,28 @@ def test_ordinary_calls_are_the_glues(cqt):
     xg = x.clone().requires_grad_(True)
     t.bwd(*t.fwd(xg)).sum().backward()
     assert t._glue.fwd(xg) is not None
+
+
+def test_both_paths_launch_one_direction_at_a_time(cqt):
+    """The two paths share the engine's buffers: while a direction's launches are
+    held together, neither path launches another; mixed threads on one stream
+    give every caller its own result."""
+    import threading
+    from concurrent.futures import ThreadPoolExecutor
+    from flash_cqt.trainable import TrainableCQT
+    t = _engine(cqt, "glue")
+    twin = TrainableCQT.__new__(TrainableCQT)              # the Python path on the same engine
+    twin.__dict__.update(t.__dict__, _glue=None)
+    xs = [_x(2, seed=i) for i in range(4)]
+    want = [t.bwd(*t.fwd(x)) for x in xs]
+    for e in (t, twin):
+        done = threading.Event()
+        with t.f._launching:
+            worker = threading.Thread(target=lambda: (e.fwd(xs[0]), done.set()))
+            worker.start()
+            assert not done.wait(0.3)
+        assert done.wait(30)
+        worker.join()
+    with ThreadPoolExecutor(8) as pool:
+        got = list(pool.map(lambda i: (t, twin)[i % 2].bwd(*(t, twin)[i // 2 % 2].fwd(xs[i % 4])), range(64)))
+    assert all(torch.equal(y, want[i % 4]) for i, y in enumerate(got))
