@@ -97,7 +97,7 @@ static void launch_route(int64_t ntasks, int64_t batch, hipStream_t stream, cons
                       kBandSliceMajorMinBatch <= kBandWriteThroughMaxBatch,
                   "batch ranges: plain task-major, write-through task-major, write-through slice-major, "
                   "plain slice-major");
-    const bool past = LAYOUT == kSliced ? stream_sliced_coef(total, ncoef)
+    const bool past = LAYOUT == kSliced ? total >= kStreamSlicedCoefMinBatch
                       : LAYOUT == FCQT_INTERLEAVED ? total >= kStreamInterleavedMinBatch : stream_planes_out(total, ncoef);
     if (past)
         hipLaunchKernelGGL((k_route_bands<LAYOUT, Store::kStream, true>), grid, dim3(kBandThreads), 0, stream, xs, cre,
@@ -121,7 +121,7 @@ static void launch_scatter(int64_t ntasks, int64_t batch, hipStream_t stream, co
                            float* f, const int2* scat, const int4* tasks, long ncoef, const SliceMap& sm,
                            const float2* tws) {
     const dim3 grid((unsigned)(ntasks * batch));
-    const bool past = LAYOUT == kSliced ? stream_sliced_coef(batch, ncoef)
+    const bool past = LAYOUT == kSliced ? batch >= kStreamSlicedCoefMinBatch
                       : LAYOUT == FCQT_INTERLEAVED ? batch >= kStreamInterleavedMinBatch : stream_planes_in(batch, ncoef);
     if (past)
         hipLaunchKernelGGL((k_scatter_bands<LAYOUT, Store::kPlain, true, true>), grid, dim3(kBandThreads), 0, stream,

@@ -76,12 +76,15 @@ static_assert(kAnalysisChunk == 128 && kAnalysisChunkMinBatch == 256, "chunk con
 //   A fwd 384 188.9 / 190.7, 512 263.9 / 262.2, rt 320 364.0 / 360.3, 512 566.0 / 567.4)
 //     A rt   192 196.6 / 196.2  224 227.4 / 227.3  256 268.6 / 262.8   320 333.6 / 319.6
 //     B rt   192 183.8 / 183.6  224 205.1 / 204.0  256 235.8 / 233.4   320 299.7 / 286.3
-//   SlicedCQT's coefficients (a new buffer on each call, both ends), a round trip's
-//   buffers of 340 MB (A 126 slices, B 140)
-//     A rt   105 120.5 / 126.7  120 132.7 / 137.1  128 143.4 / 139.9   144 181.3 / 165.0
-//     A fwd  105 54.1 / 56.8    120 60.1 / 62.2    126 64.4 / 61.7     144 80.4 / 76.1
-//     B rt   105 108.2 / 113.3  120 116.8 / 123.3  136 143.6 / 141.6   160 177.4 / 163.8
-//     B fwd  120 51.9 / 53.7    136 64.0 / 64.0    140 63.4 / 65.2     144 71.2 / 66.8
+//   SlicedCQT's coefficients (a new buffer on each call), written and read, 105 slices;
+//   in a loop that keeps its last result, and, dropping it before the next call, so that
+//   the allocator hands the same block out again
+//     A rt   104 136.5 / 124.2  120 147.8 / 136.7  136 167.8 / 157.2   144 181.2 / 163.8
+//       dropped: 118.2 / 124.1      133.8 / 136.8      160.3 / 157.0       180.0 / 163.7
+//     A fwd  104 60.8 / 54.5    120 66.0 / 59.9    136 77.4 / 72.5     144 81.1 / 74.0
+//       dropped: 52.6 / 55.0        59.5 / 60.1        74.3 / 72.7         78.3 / 74.4
+//     B rt   104 122.1 / 110.5  120 128.2 / 122.0  136 149.3 / 142.3   144 160.8 / 147.8
+//       dropped: 104.5 / 111.2      116.3 / 122.2      138.5 / 141.6       151.7 / 148.1
 //   SlicedCQT's output, kStreamYMinBatch: rt 120 137.6 / 135.7, 160 184.3 / 178.3, 224 246.4 /
 //   239.2, bwd 512 304.4 / 292.1. Its signals are read twice (the overlap) and not streamed.
 constexpr int64_t kStreamXMinBatch = 124;
@@ -90,22 +93,15 @@ constexpr int64_t kStreamPlanesInBytes = 259000000;
 constexpr int64_t kStreamPlanesOutBytes = 353600000;
 constexpr int64_t kStreamInterleavedMinBatch = 140;
 constexpr int64_t kStreamWMinBatch = 192;
-constexpr int64_t kStreamSlicedCoefBytes = 340000000;
+constexpr int64_t kStreamSlicedCoefMinBatch = 105;
 
-// Bytes of x, W, X and the coefficients, and of a round trip's buffers (F and y
-// too), for a call of `batch` slices.
+// Bytes of x, W, X and the coefficients of a call of `batch` slices.
 inline int64_t analysis_bytes(int64_t batch, int64_t ncoef) { return batch * (4 * FCQT_N + 16 * FCQT_L + 8 * ncoef); }
-inline int64_t round_trip_bytes(int64_t batch, int64_t ncoef) {
-    return analysis_bytes(batch, ncoef) + batch * (8 * FCQT_FROW + 4 * FCQT_N);
-}
 inline bool stream_planes_in(int64_t batch, int64_t ncoef) {
     return analysis_bytes(batch, ncoef) >= kStreamPlanesInBytes;
 }
 inline bool stream_planes_out(int64_t batch, int64_t ncoef) {
     return analysis_bytes(batch, ncoef) >= kStreamPlanesOutBytes;
-}
-inline bool stream_sliced_coef(int64_t batch, int64_t ncoef) {
-    return round_trip_bytes(batch, ncoef) >= kStreamSlicedCoefBytes;
 }
 
 inline bool aligned(const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }

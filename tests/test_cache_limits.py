@@ -24,8 +24,7 @@ def _first(tmp_path, rule):
     return tuple(map(int, subprocess.run([str(exe)], check=True, capture_output=True, text=True, timeout=60).stdout.split()))
 
 
-@pytest.mark.parametrize("rule,first", [("stream_sliced_coef(batch, ncoef)", (126, 140)),
-                                        ("stream_planes_in(batch, ncoef)", (140, 165)),
+@pytest.mark.parametrize("rule,first", [("stream_planes_in(batch, ncoef)", (140, 165)),
                                         ("stream_planes_out(batch, ncoef)", (192, 224))])
 def test_first_batch_past_the_caches(tmp_path, rule, first):
     assert _first(tmp_path, rule) == first
