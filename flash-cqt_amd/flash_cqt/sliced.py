@@ -314,9 +314,8 @@ class SlicedCQT:
         base = parts[0]._base
         if side is not None and base is not None and base.dim() == 1 and base.dtype == torch.complex64 \
                 and base.numel() == nsig * S * f.ncoef and base.device == f.dev and base.is_contiguous():
-            ptr = base.data_ptr()
-            if all(p._base is base and p.is_contiguous() and p.data_ptr() == ptr + 8 * nsig * S * off
-                   and not p.is_conj() and not p.is_neg()
+            ptr, row = base.data_ptr(), 8 * nsig * S
+            if all(p._base is base and p.is_contiguous() and not p.is_conj() and p.data_ptr() == ptr + row * off
                    for p, (_, _, off) in zip(parts, f.gspec)):
                 return base
         coef = torch.zeros(nsig * S * f.ncoef, dtype=torch.complex64, device=f.dev)

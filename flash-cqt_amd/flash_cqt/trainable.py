@@ -15,6 +15,8 @@ returned blocks are views into it (no per-group copies), and bwd reads that
 buffer in place when it is handed the same views back (the reference
 concatenates the blocks, trainable.py:161-164).
 """
+import operator
+
 import torch
 
 from . import _native
@@ -49,11 +51,7 @@ class TrainableCQT:
     def _own_directions(self):
         """No direction replaced, by a subclass, on the class or on this object:
         the glue would pass such a method by."""
-        cls = type(self)
-        for name, own in _DIRECTIONS:
-            if getattr(cls, name) is not own:
-                return False
-        return self.__dict__.keys().isdisjoint(_NAMES)
+        return _directions(type(self)) == _OWN and self.__dict__.keys().isdisjoint(_NAMES)
 
     # ------------------------------------------------ engine directions
     # The inputs reaching these are [B, N] float32 or [B, ncoef] complex64,
@@ -183,7 +181,8 @@ class TrainableCQT:
 # the methods that the host glue stands in for
 _NAMES = ("_launch_analysis", "_launch_synthesis", "_analysis", "_synthesis", "_adj_analysis", "_adj_synthesis",
           "_base_of")
-_DIRECTIONS = tuple((n, getattr(TrainableCQT, n)) for n in _NAMES)
+_directions = operator.attrgetter(*_NAMES)
+_OWN = _directions(TrainableCQT)
 
 
 class _Analysis(torch.autograd.Function):
