@@ -43,9 +43,13 @@ static_assert(kAnalysisChunk == 128 && kAnalysisChunkMinBatch == 256, "chunk con
 //     A bwd  105 65.1 / 63.9    120 70.8 / 70.6    144 83.9 / 83.9
 //     B rt   105 102.8 / 99.9   120 116.7 / 111.8  136 130.7 / 125.9   200 180.5 / 176.8
 //     B bwd  105 58.9 / 57.6    120 64.0 / 64.2    144 77.6 / 77.7
-//     training steps, whose loss reads y: A 105 304.8 / 305.2, 112 318.5 / 324.1,
-//     124 353.0 / 348.5, 136 387.0 / 394.0, 144 389.9 / 388.2; B 112 287.2 / 286.6,
-//     127 318.8 / 325.7, 136 347.8 / 354.4, 144 356.0 / 355.0 (-1.5 to +2%)
+//     TrainableCQT's y is a new buffer on each call, which a loss reads at once; steps take
+//     -1.4 to +2.7% by it (loops that keep their last result), round trips without gradients
+//     gain 2-4% where the last result is dropped and lose up to 5% where it is kept:
+//     A step 105 313.7 / 311.6  120 345.2 / 351.5  128 351.8 / 355.7   136 391.2 / 401.7
+//     B step 105 289.5 / 285.3  120 315.8 / 319.7  128 324.3 / 331.6   136 350.7 / 355.7
+//     A rt, kept 112 125.7 / 129.9   128 137.5 / 142.1   136 154.5 / 163.5   144 153.8 / 153.5
+//     A rt, dropped  122.5 / 117.9       131.8 / 129.3       147.4 / 143.1       153.6 / 153.2
 //   coefficient planes read by the scatter, x + W + X + planes of 259 MB: the planes
 //   just written no longer outlive the rest of the analysis (A 140 slices, B 165)
 //     A rt   132 146.2 / 144.5  144 159.5 / 155.0  152 170.6 / 164.1   160 188.2 / 169.8
@@ -71,6 +75,7 @@ static_assert(kAnalysisChunk == 128 && kAnalysisChunkMinBatch == 256, "chunk con
 //     A rt   132 142.5 / 143.3  140 149.9 / 148.8  160 170.6 / 164.9   172 182.8 / 175.7
 //     B step 132 340.5 / 335.8  140 353.8 / 346.6  160 386.9 / 382.2   172 415.8 / 413.8
 //     B rt   132 121.1 / 123.9  140 133.4 / 133.5  160 149.4 / 146.7   172 162.0 / 157.7
+//   (loops that drop each result; one that keeps its last gains at every size from 105 on)
 //   W read by the row pass, 192 slices of a whole call (in the 128-slice chunks of
 //   fcqt_sliced_analysis, whose W was written just before, either form is within 1%:
 //   A fwd 384 188.9 / 190.7, 512 263.9 / 262.2, rt 320 364.0 / 360.3, 512 566.0 / 567.4)
