@@ -296,13 +296,18 @@ def inv_col(w, c, cpw=32):
 US128 = Plan(128).US
 
 
+AHEAD = 128                      # fold-list entries whose slots load ahead of them
+
+
 def col_inv_stage(Fs, fold, w, cpw=32):
     """LDS of inverse column workgroup w (CPW columns) after its staging
     phase, by the kernel's own arithmetic: slot c holds column
     inv_col(w, c) at [c US + n1] (plane sum), bin L at [128] of slot 0 in
     workgroup 0, and each fold-list entry of the containing wide list is
-    added at the position the kernel computes, if this workgroup owns it.
-    Returns (lds, entries used)."""
+    added at the position the kernel computes, if this workgroup owns it. A
+    thread's first entry takes the slots loaded ahead of it where its overflow
+    index is its place in the lists (counted in col_inv_stage.ahead), any
+    other loads them after it. Returns (lds, entries used)."""
     h = cpw // 2
     nthreads = 8 * cpw
     share = (256 // cpw) // FOLD_LISTS
@@ -319,6 +324,12 @@ def col_inv_stage(Fs, fold, w, cpw=32):
     used = []
     lst = fold[(w // share) * T.FOLD_PER_WG:(w // share + 1) * T.FOLD_PER_WG]
     for tid in range(nthreads):
+        at = (w // share) * T.FOLD_PER_WG + tid
+        slots = None
+        if tid < AHEAD:
+            o = 2 * T.FSTRIDE + 2 * at
+            assert o % 2 == 0 and o + 2 <= T.FROW      # one 16-byte load inside the row
+            slots = Fs[o:o + 2]
         for e in range(nent):
             ent = int(lst[tid + e * nthreads])
             if ent < 0:
@@ -337,10 +348,17 @@ def col_inv_stage(Fs, fold, w, cpw=32):
             if pos >= 0:
                 assert 0 <= pos < cpw * US128
                 k = min(ent >> 16, T.OVF_CAP - 1)
-                o = 2 * T.FSTRIDE + 2 * k
-                lds[pos] += Fs[o] + Fs[o + 1]
+                if e == 0 and slots is not None and k == at:
+                    lds[pos] += slots[0] + slots[1]
+                    col_inv_stage.ahead += 1
+                else:
+                    o = 2 * T.FSTRIDE + 2 * k
+                    lds[pos] += Fs[o] + Fs[o + 1]
                 used.append(ent)
     return lds, used
+
+
+col_inv_stage.ahead = 0
 
 
 def packed_fft_inv(F, ovf=None, shape=WIDE):
@@ -592,44 +610,102 @@ def overlap_add(y, nsig, S, length, vec4=False):
     return out
 
 
-def row_inv_ola(y, nsig, S, length):
-    """The inverse row pass with the overlap-add fused into its store
-    (k_row_inv_ola): a launch over the even slices, then one over the odd
-    slices. Slice s's sample jj goes to p = 2H (s - 1) + j, j = (jj + H) mod N
-    (even s) or (jj - H) mod N (odd s), if 0 <= p < length. Even slices store
-    0 + v; odd slices add to what the even launch stored, except in their
-    second half when no slice s + 1 exists, where they store 0 + v. Asserts
-    every output sample is stored exactly once before it is added to, and at
-    most once added to, in launch order."""
-    H = N // 4
-    hop = 2 * H
+OLA_RUN = 4096                   # samples between a thread's pairs of a slice
+
+
+def ola_hops(total):
+    """Hops per tile of the overlap-adding row pass (packed_fft.hip ola_hops)."""
+    return 1 if total < 160 else 2 if total < 320 else 4
+
+
+def ola_lanes(rpw):
+    """First sample of each thread's pair u = 0, over the row tiles and threads
+    of a slice: lane = 2 (rg RPW + (tid mod RPW) + 128 (tid / RPW))."""
+    rg, tid = np.meshgrid(np.arange(128 // rpw), np.arange(16 * rpw), indexing="ij")
+    lanes = (2 * (rg * rpw + (tid & (rpw - 1)) + 128 * (tid // rpw))).reshape(-1)
+    assert np.array_equal(np.sort(lanes), np.arange(0, OLA_RUN, 2))
+    return lanes
+
+
+def _pairs(row, lanes, u):
+    """The sample pairs u of every thread of one inverse slice [N], [threads, 2]."""
+    return np.stack([row[lanes + OLA_RUN * u], row[lanes + OLA_RUN * u + 1]], -1)
+
+
+def _halves(s):
+    """u of run 0 of slice s's first and second half."""
+    return (4, 12) if s & 1 else (12, 4)
+
+
+def row_inv_ola(y, nsig, S, length, rpw=16, hops=None):
+    """The inverse row pass with the overlap-add in its store (k_row_inv_ola)
+    on inverse slices y [nsig * S, N]: tiles of `hops` consecutive hops walk
+    slices h0 .. min(h1, S - 1), a thread keeps the eight pairs of a slice's
+    second half, adds the next slice's first half and stores pairs, or single
+    samples where the row ends between two. Asserts that the slice loaded ahead
+    is in range and next, and that every output sample is stored exactly once."""
+    hop = N // 2
+    nhops = -(-length // hop)
+    assert 1 <= nhops <= S
+    hops = ola_hops(nsig * nhops) if hops is None else hops
     out = np.full((nsig, length), np.nan, np.float32)
     stored = np.zeros((nsig, length), np.int64)
-    added = np.zeros((nsig, length), np.int64)
-    jj = np.arange(N)
-    for odd in (0, 1):
-        for sig in range(nsig):
-            for s in range(odd, S, 2):
-                j = (jj + (N - H if odd else H)) & (N - 1)
-                p = hop * (s - 1) + j
-                ok = (p >= 0) & (p < length)
-                v = y[sig * S + s][ok].astype(np.float32)
-                pp = p[ok]
-                if odd:
-                    add = (j[ok] < hop) | (s + 1 < S)
-                    assert (stored[sig, pp[add]] == 1).all() and (added[sig, pp[add]] == 0).all()
-                    out[sig, pp[add]] = out[sig, pp[add]] + v[add]
-                    added[sig, pp[add]] += 1
-                    st = ~add
-                    assert (stored[sig, pp[st]] == 0).all()
-                    out[sig, pp[st]] = np.float32(0) + v[st]
-                    stored[sig, pp[st]] += 1
-                else:
-                    assert (stored[sig, pp] == 0).all()
-                    out[sig, pp] = np.float32(0) + v
-                    stored[sig, pp] += 1
+    lanes = ola_lanes(rpw)
+
+    def store(sig, p, v, pair, single):
+        for ok, n in ((pair, 2), (single, 1)):
+            for k in range(n):
+                q = p[ok] + k
+                assert (q >= 0).all() and (q < length).all()
+                out[sig, q] = v[ok, k]
+                stored[sig, q] += 1
+
+    for sig in range(nsig):
+        for h0 in range(0, nhops, hops):
+            h1 = min(h0 + hops, nhops)
+            last = min(h1, S - 1)
+            ahead, carry, s = h0, None, h0
+            while True:
+                assert ahead == s <= last < S
+                row = y[sig * S + s].astype(np.float32)
+                ahead = min(s + 1, last)
+                first, second = _halves(s)
+                base = hop * (s - 1) + lanes
+                room = length - base
+                kept = []
+                for i in range(8):
+                    v, w = _pairs(row, lanes, (first + i) & 15), _pairs(row, lanes, (second + i) & 15)
+                    if s > h0:
+                        store(sig, base + OLA_RUN * i, carry[i] + v, room >= OLA_RUN * i + 2, room == OLA_RUN * i + 1)
+                    kept.append(np.float32(0) + w)
+                carry = kept
+                if s == last:
+                    break
+                s += 1
+            if h1 == S:
+                p = hop * last + lanes
+                for i in range(8):
+                    q = p + OLA_RUN * i
+                    store(sig, q, carry[i], q + 1 < length, q + 1 == length)
     assert (stored == 1).all()
     return out
+
+
+def row_inv_stream(y, tail, k, rpw=16):
+    """k_row_inv_stream on inverse slices k, y [nsig, N] and tail [nsig, N / 2]:
+    (out or None, new tail), each position read and replaced by one thread."""
+    lanes = ola_lanes(rpw)
+    first, second = _halves(k)
+    out, new = np.full_like(tail, np.nan), np.full_like(tail, np.nan)
+    for sig in range(y.shape[0]):
+        for i in range(8):
+            p = lanes + OLA_RUN * i
+            v, w = _pairs(y[sig], lanes, (first + i) & 15), _pairs(y[sig], lanes, (second + i) & 15)
+            for e in range(2):
+                out[sig, p + e] = tail[sig, p + e] + v[:, e]
+                new[sig, p + e] = w[:, e]
+    assert not np.isnan(new).any()
+    return (out if k > 0 else None), new
 
 
 def stream_overlap(y, tail, k):

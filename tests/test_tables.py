@@ -239,15 +239,16 @@ def test_overlap_add_index_math_cpu():
             assert np.array_equal(ks.overlap_add(y, 2, S, length, vec4=True), ref)
 
 
-def test_fused_row_overlap_add_index_math_cpu():
-    """The inverse row pass with the overlap-add in its store (even slices,
-    then odd ones) writes every output sample once before adding to it, and
-    gives k_overlap_add's bits, signed zeros included, for ragged lengths,
-    one slice, and slices past the end of the signal."""
+@pytest.mark.parametrize("rpw,hops", [(16, None), (8, 1), (16, 2), (8, 4), (16, 3)])
+def test_fused_row_overlap_add_index_math_cpu(rpw, hops):
+    """The inverse row pass with the overlap-add in its store (tiles of hops,
+    second halves carried) stores every output sample once and gives
+    k_overlap_add's bits, signed zeros included, for ragged lengths, tiles that
+    end inside a signal, one slice, and slices past the end of the signal."""
     N, H = ks.N, ks.N // 4
     rs = np.random.RandomState(6)
     cases = [(8, None), (1000, None), (3 * 2 * H + 12, None), (5 * 2 * H, None), (2 * H - 2, None),
-             (1000, 1), (2 * H, 1), (2 * H + 1, 2), (7, 5)]
+             (1000, 1), (2 * H, 1), (2 * H + 1, 2), (7, 5), (5 * 2 * H - 4097, 6), (4 * 2 * H, 4)]
     for length, S in cases:
         if S is None:
             quarters = -(-length // H)
@@ -256,8 +257,50 @@ def test_fused_row_overlap_add_index_math_cpu():
         y[:, ::97] = np.float32(-0.0)                 # exact zeros of both signs
         y[:, 1::89] = np.float32(0.0)
         ref = ks.overlap_add(y, 2, S, length)
-        got = ks.row_inv_ola(y, 2, S, length)
+        got = ks.row_inv_ola(y, 2, S, length, rpw=rpw, hops=hops)
         assert np.array_equal(got.view(np.uint32), ref.view(np.uint32)), (length, S)
+
+
+@pytest.mark.parametrize("rpw", [8, 16])
+def test_fused_stream_overlap_index_math_cpu(rpw):
+    """The streamed row pass replaces its tail as k_stream_overlap does."""
+    rs = np.random.RandomState(7)
+    tail = np.zeros((2, ks.N // 2), np.float32)
+    for k in range(4):
+        y = rs.standard_normal((2, ks.N)).astype(np.float32)
+        ref, got = ks.stream_overlap(y, tail, k), ks.row_inv_stream(y, tail, k, rpw=rpw)
+        assert (got[0] is None) == (k == 0) and (k == 0 or np.array_equal(got[0], ref[0]))
+        assert np.array_equal(got[1], ref[1])
+        tail = ref[1]
+
+
+@pytest.mark.parametrize("cpw", [16, 32])
+def test_overflow_slots_loaded_ahead_cpu(factored_tables, cpw):
+    """The column pass stages the same sums from the slots loaded ahead of a
+    fold list's entries as from those loaded after them (indices numbered by
+    ascending bin, as other builders may)."""
+    from flash_cqt import tables as T
+    from test_gpu_fold_order import _in_bin_order
+    t = factored_tables
+    u = _in_bin_order(t, T)
+    rs = np.random.RandomState(8)
+    vals = rs.standard_normal(T.FROW) + 1j * rs.standard_normal(T.FROW)
+    for name in ("ovf_scat", "ovf_scat_a"):
+        Fs, Fu = vals.copy(), vals.copy()
+        at = np.flatnonzero(t[name] >= 0)
+        where = {int(b) & 0xFFFF: int(b) >> 16 for b in u[name][u[name] >= 0]}
+        for e in t[name][at].tolist():
+            o, q = (2 * T.FSTRIDE + 2 * k for k in (e >> 16, where[e & 0xFFFF]))
+            Fu[q:q + 2] = Fs[o:o + 2]
+        ahead, total = [], 0
+        for F, tab in ((Fs, t), (Fu, u)):
+            ks.col_inv_stage.ahead = 0
+            got = [ks.col_inv_stage(F, tab[name], w, cpw) for w in range(256 // cpw)]
+            ahead.append(ks.col_inv_stage.ahead)
+            if F is Fs:
+                ref, total = got, sum(len(used) for _, used in got)
+        assert total == at.size and ahead[0] == np.count_nonzero(at % T.FOLD_PER_WG < ks.AHEAD) > ahead[1]
+        assert all(np.array_equal(a[0], b[0], equal_nan=True) for a, b in zip(ref, got))
 
 
 def test_stream_overlap_index_math_cpu():
