@@ -434,7 +434,7 @@ __device__ __forceinline__ void row_fwd_tile(const int b, const int w, const flo
 }
 
 
-template <int RPW, Store S, bool STREAM = false>
+template <int RPW, Store S>
 __device__ __forceinline__ void row_inv_tile(const int b, const int rg, const float2* __restrict__ in,
                                              float2* __restrict__ y, const float2* __restrict__ tws, float2* lds,
                                              const int tid = threadIdx.x) {
@@ -442,7 +442,7 @@ __device__ __forceinline__ void row_inv_tile(const int b, const int rg, const fl
     float2* tw2 = lds + RPW * P::US;
     const int rho = tid >> 4;
     const int t = tid & 15;
-    row_fft_to_lds<false, STREAM>(in + (long)b * kL + (long)(rg * RPW + rho) * 256, lds, tw2, rho, t, 16 * RPW, tws,
+    row_fft_to_lds<false, false>(in + (long)b * kL + (long)(rg * RPW + rho) * 256, lds, tw2, rho, t, 16 * RPW, tws,
                           nullptr, nullptr, tid);
     const int rho2 = tid & (RPW - 1);
     const int kg = tid / RPW;
@@ -468,10 +468,10 @@ __device__ __forceinline__ void row_inv_tile(const int b, const int rg, const fl
 // A thread's 16 sample pairs of a slice lie at j = lane + 4096 u, lane = 2 (kk1 +
 // 128 kg) < 4096, and the quarter roll moves whole runs of 4096: pair u goes to
 // run (u + 4) mod 16 of the slice in even slices and (u + 12) mod 16 in odd
-// ones. So run i of a hop is u = i + 4 (mod 16, kHigh) or u = i + 12 (kLow) of
-// the same thread in every slice: it keeps a slice's second half in registers,
-// adds the next slice's first half and stores each output sample once, and no
-// slice ever goes to memory. Slice h1 is transformed again by the next tile of
+// ones. So run i of a slice's first half is u = i + 12 (mod 16) in even slices and
+// i + 4 in odd ones, of its second half the other, of the same thread in every
+// slice: it keeps a slice's second half in registers, adds the next slice's first
+// half and stores each output sample once, and no slice ever goes to memory. Slice h1 is transformed again by the next tile of
 // the signal (its second half), so a tile of k hops costs k + 1 slices; the next
 // slice's rows are loaded while this one is transformed. The sums are
 // k_overlap_add's: (0 + a) + b of the rounded products k_row_inv stores.

@@ -36,12 +36,12 @@ from .ref_util import hann_fft_order
 from .oct_cqt import OctCQT
 
 
-# From this many slices on the whole-signal synthesis overlap-adds in the
-# inverse row pass (fcqt_sliced_synthesis); below, the slices go through a
-# slice buffer and one overlap-add kernel. The row pass measured faster at
-# every size (SlicedCQT.bwd, fused against buffered): 23 against 32 us up to 15
-# slices, 75.6 against 79.3 us at 120 and 127 against 142 us at 224. Same
-# bits either way.
+# From this many slices on, always, the whole-signal synthesis overlap-adds in
+# the inverse row pass (fcqt_sliced_synthesis). Below, the slices go through a
+# slice buffer and one overlap-add kernel, with the same bits: the benchmark and
+# the GPU tests raise the constant to compare the two. The row pass measured
+# faster at every size (SlicedCQT.bwd, fused against buffered): 23 against 32 us up to 15
+# slices, 75.6 against 79.3 us at 120 and 127 against 142 us at 224.
 FUSED_OLA_MIN_SLICES = 1
 
 
@@ -226,9 +226,9 @@ class SlicedCQT:
         (x="chunk": the whole-signal analysis, which from 256 slices on runs
         in chunks of 128 slices through the same leading rows, so X holds
         sliced_analysis_rows rows; x="full": one row per slice, the streamed
-        analysis; x=False: none), and with y=True (the streamed synthesis) a
-        slice buffer Y; the whole-signal synthesis overlap-adds inside its
-        row pass and needs neither X nor Y. There is one
+        analysis; x=False: none), and with y=True a slice buffer Y (only the
+        slice-buffer inverse below FUSED_OLA_MIN_SLICES: the others overlap-add
+        inside the row pass). There is one
         buffer set per engine, sized to the largest row count seen so far
         (X and Y to the largest that asked for them); a smaller call uses
         leading rows. Rows are independent, and F is only ever used with the
@@ -394,7 +394,7 @@ class SlicedCQT:
         bufs, cache = self._caches(f)
         st = cache.get(nsig)
         if st is None:
-            st = {k: v.data_ptr() for k, v in self._ws(f, nsig, 1, y=True, x="full").items()}
+            st = {k: v.data_ptr() for k, v in self._ws(f, nsig, 1, x="full").items()}
             st["tw"] = self._tw32().data_ptr()
             cache[nsig] = st
         elif torch.cuda.is_current_stream_capturing():
@@ -528,7 +528,7 @@ class SlicedCQT:
                 # scatter, inverse passes and the half-slice overlap-add in one call
                 _native.check(f.lib.fcqt_stream_synthesis(f._ct, f._tp["scat"], f._tp["slice_groups"],
                                                           f._tp["ovf_scat"], coef.data_ptr(), st["F"], st["W"],
-                                                          st["Y"], tail.data_ptr(),
+                                                          st["W"], tail.data_ptr(),     # its y: not used
                                                           out.data_ptr() if out is not None else None, nsig, k,
                                                           _native.stream_handle(f.dev.index)), "stream_synthesis")
                 if out is not None:

@@ -438,9 +438,9 @@ int fcqt_stream_analysis(const fcqt_tables* tab, const int32_t* route, const int
 
 /* One streamed synthesis step: fcqt_scatter_bands_sliced (one slice per
  * signal, first = slice), the inverse passes and the sums of
- * fcqt_stream_overlap in the row pass's store (y, a slice buffer as that call
- * takes, is required but not used), with every argument checked before the
- * first launch. out may be NULL for slice 0.
+ * fcqt_stream_overlap in the row pass's store (y, which that call
+ * takes, is required but not used: any pointer of its alignment, work's say),
+ * with every argument checked before the first launch. out may be NULL for slice 0.
  * Replaces the per-slice step of SlicedCQT.stream_bwd (sliced.py:194-209):
  * _arrange, inv_bands, inv_tail, the roll and the half-slice overlap-add. */
 int fcqt_stream_synthesis(const fcqt_tables* tab, const int32_t* scat, const int32_t* groups,

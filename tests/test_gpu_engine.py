@@ -737,10 +737,10 @@ def test_sliced_chunked_analysis_same_bits(fused, nsig, S):
 @pytest.mark.parametrize("nsig,S,length", [(1, 1, 1000), (3, 5, 7), (2, 20, 17 * 32768 + 3), (2, 4, 2 * 32768),
                                            (8, 15, 441000), (1, 2, 32769), (4, 40, 39 * 32768 + 100)])
 def test_sliced_synthesis_fused_overlap_add_same_bits(fused, nsig, S, length):
-    """fcqt_sliced_synthesis (even slices stored, odd slices added, in the
-    inverse row pass's store) gives the bits of scatter + inverse passes +
-    k_overlap_add, signed zeros included: one slice, slices past the end of
-    a short output, odd lengths (4-byte stores) and even ones (8-byte)."""
+    """fcqt_sliced_synthesis (second halves carried from slice to slice in the
+    inverse row pass, every sample stored once) gives the bits of scatter +
+    inverse passes + k_overlap_add, signed zeros included: one slice, slices
+    past the end of a short output, odd lengths and even ones."""
     rs = np.random.RandomState(19)
     B = nsig * S
     coef = torch.from_numpy((rs.standard_normal((B * fused.ncoef,)) + 1j * rs.standard_normal((B * fused.ncoef,)))
@@ -761,8 +761,8 @@ def test_sliced_synthesis_fused_overlap_add_same_bits(fused, nsig, S, length):
 
 
 def test_sliced_long_signals_round_trip():
-    """SlicedCQT on 2 x 160 slices (the chunked analysis and, from 256
-    slices on, the overlap-add in the row pass): round trip >= 125 dB, and
+    """SlicedCQT on 2 x 160 slices (the chunked analysis and the overlap-add
+    in the row pass): round trip >= 125 dB, and
     the inverse equal to the slice-buffer path's (scatter, inverse passes,
     overlap-add kernel) bit for bit."""
     from flash_cqt import SlicedCQT

@@ -369,7 +369,7 @@ def test_sliced_buffer_sets_kept_for_recorded_graphs_cpu(monkeypatch):
     third_call = s._ws(f, 2, 2)                          # grows again
     assert s._fused_ws["recorded"] == [second] and s._fused_ws["rows"]["B"] == 4
     assert "Y" not in third_call and "Y" not in s._fused_ws["rows"]   # the whole-signal path needs no Y
-    assert s._ws(f, 3, 1, y=True)["Y"].shape == (3, T.N)           # the streamed synthesis gets one
+    assert s._ws(f, 3, 1, y=True)["Y"].shape == (3, T.N)           # a call that asks for one
     y3 = s._fused_ws["rows"]["Y"]
     capturing[0] = True
     s._ws(f, 3, 1, y=True)
