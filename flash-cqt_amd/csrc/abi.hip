@@ -19,8 +19,8 @@ __global__ __launch_bounds__(256) void k_fill_zero(float4* __restrict__ p4, long
 // still spread over the chip (16-byte accesses where both ends allow them).
 // Graphed returns its outputs with it: a B = 1 round trip's planes and signal
 // (1.3 MB) in one launch instead of three copies by the runtime, the whole call
-// 54.1 -> 43.9 us (torch's foreach copy, 64 Ki elements per workgroup, was slower
-// than the three copies).
+// 49-54 -> 42-45 us over four cards (torch's foreach copy, 64 Ki elements per
+// workgroup, was slower than the three copies).
 constexpr int64_t kCopyPerWg = FCQT_COPY_SHARE;
 struct CopyArgs {
     const char* src[FCQT_COPY_MAX];

@@ -230,9 +230,11 @@ __device__ __forceinline__ void col_inv_tile(const int b, const int w, const flo
     // The overflow slots of the list's first kAhead entries, loaded before the
     // entries arrive: the builder gives entry e of list l the index l kFoldPerWg
     // + e. Any other entry or index (other builders' images) loads its slots
-    // after it. One memory latency less on the pass's critical path: synthesis
-    // at B = 1 / 4 / 16 / 64 14.0 / 14.9 / 18.3 / 38.0 -> 13.8 / 14.6 / 18.1 /
-    // 37.5 us (without any overflow slots 13.4 / 14.2 / 17.7 / 37.2).
+    // after it. One memory latency less on the pass's critical path, little beside
+    // a direction's launches: synthesis at B = 1 / 4 / 8 / 16 / 32 / 64 14.0 / 14.7 / 15.9 /
+    // 18.8 / 25.0 / 45.4 -> 13.7 / 14.5 / 15.6 / 18.6 / 24.9 / 44.9 us, 105 65.8 -> 65.1; from
+    // about 110 slices on, where the extra 16 KB of a slice are traffic, a wash (127 79.2
+    // / 79.3, round trips 133.7 / 134.5, 512 519.4 / 519.2).
     constexpr int kAhead = 128;
     const int ahead = (w / kShare) * kFoldPerWg + tid;      // the index of this thread's entry 0
     float4 slots = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
