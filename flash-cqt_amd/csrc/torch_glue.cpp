@@ -178,15 +178,18 @@ bool plain_call() {
            c10::hip::currentStreamCaptureStatusMayInitCtx() == c10::hip::CaptureStatus::None;
 }
 
-// A strided tensor of the given GPU and type, no lazy conjugation or
-// negation, no tangent.
-bool plain_tensor(const c10::Device& device, const Tensor& t, at::ScalarType type) {
+// No subclass, wrapper, lazy conjugation or negation: its values are its memory.
+bool own_values(const Tensor& t) {
     static const c10::DispatchKeySet odd({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchBatched,
                                           c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::Functionalize,
                                           c10::DispatchKey::Conjugate, c10::DispatchKey::Negative,
                                           c10::DispatchKey::ZeroTensor});
-    return t.defined() && !t.key_set().has_any(odd) && t.layout() == c10::kStrided && t.device() == device &&
-           t.scalar_type() == type && !t._fw_grad(0).defined();
+    return t.defined() && !t.key_set().has_any(odd) && t.layout() == c10::kStrided;
+}
+
+// A strided tensor of the given GPU and type with values of its own, no tangent.
+bool plain_tensor(const c10::Device& device, const Tensor& t, at::ScalarType type) {
+    return own_values(t) && t.device() == device && t.scalar_type() == type && !t._fw_grad(0).defined();
 }
 
 // (octave blocks, side blocks) of x [..., N], or None
@@ -239,6 +242,25 @@ Tensor base_of(const Engine& e, const std::vector<Tensor>& parts, int64_t batch)
         if (c.stride(-1) != 1 || (g.bands != 1 && c.stride(-2) != g.M)) return {};
     }
     return base;
+}
+
+// The flat SlicedCQT coefficient buffer of `rows` slices that the parts are all
+// the blocks of, in order, as its fwd returned them, or None.
+py::object block_base(const Ref& e, const std::vector<Tensor>& parts, int64_t rows) {
+    if (parts.size() != e->groups.size() || !own_values(parts[0]) || !parts[0].is_view()) return py::none();
+    const Tensor base(parts[0]._base());
+    if (!own_values(base) || base.device() != e->device || base.scalar_type() != at::kComplexFloat || base.dim() != 1 ||
+        base.numel() != rows * e->tab.ncoef || !base.is_contiguous())
+        return py::none();
+    const auto* ptr = static_cast<const char*>(base.data_ptr());
+    for (size_t i = 0; i < parts.size(); ++i) {
+        const Tensor& c = parts[i];
+        const Group& g = e->groups[i];
+        if (!own_values(c) || !c.is_view() || !c._base().is_same(base) || !c.is_contiguous() ||
+            c.numel() != rows * g.bands * g.M || static_cast<const char*>(c.data_ptr()) != ptr + 8 * rows * g.off)
+            return py::none();
+    }
+    return py::cast(base);
 }
 
 // y [..., N] of the blocks, or None
@@ -375,6 +397,9 @@ PYBIND11_MODULE(_fcqt_torch, m) {
         .def("__enter__", [](const Ref& e) { e->launching.lock(); }, py::call_guard<py::gil_scoped_release>())
         .def("__exit__", [](const Ref& e, const py::args&) { e->launching.unlock(); })
         .def_property_readonly("captured", [](const Ref& e) { return e->captured.load(); })
+        .def("block_base", [](const Ref& e, const std::vector<Tensor>& parts, int64_t rows) {
+            return block_base(e, parts, rows);
+        })
         .def("fwd", [](const Ref& e, const Tensor& x) { return guarded(fwd, e, x); })
         .def("bwd", [](const Ref& e, const std::vector<Tensor>& parts) { return guarded(bwd, e, parts); });
 }

@@ -311,17 +311,30 @@ class SlicedCQT:
         storage when they are the views the fused forward returned (views of
         one buffer at the group offsets), else a copy."""
         parts = list(blocks) + (list(side) if side is not None else [])
-        base = parts[0]._base
-        if side is not None and base is not None and base.dim() == 1 and base.dtype == torch.complex64 \
-                and base.numel() == nsig * S * f.ncoef and base.device == f.dev and base.is_contiguous():
-            ptr, row = base.data_ptr(), 8 * nsig * S
-            if all(p._base is base and p.is_contiguous() and not p.is_conj() and p.data_ptr() == ptr + row * off
-                   for p, (_, _, off) in zip(parts, f.gspec)):
+        if side is not None:
+            glue = None if torch.compiler.is_compiling() else getattr(f, "_glue", None)
+            base = glue.block_base(parts, nsig * S) if glue is not None else self._block_base(f, parts, nsig * S)
+            if base is not None:
                 return base
         coef = torch.zeros(nsig * S * f.ncoef, dtype=torch.complex64, device=f.dev)
         for p, (b, M, off) in zip(parts, f.gspec):
             coef[nsig * S * off:nsig * S * (off + b * M)] = p.reshape(-1).to(torch.complex64)
         return coef
+
+    @staticmethod
+    def _block_base(f, parts, rows):
+        """The buffer that the parts are all the blocks of, in order, as fwd
+        returned them, else None (the host glue's block_base in Python)."""
+        base = parts[0]._base
+        if len(parts) != len(f.gspec) or base is None or base.dim() != 1 or base.dtype != torch.complex64 \
+                or base.numel() != rows * f.ncoef or base.device != f.dev or not base.is_contiguous():
+            return None
+        ptr = base.data_ptr()
+        for p, (b, M, off) in zip(parts, f.gspec):
+            if p._base is not base or p.data_ptr() != ptr + 8 * rows * off or p.numel() != rows * b * M \
+                    or not p.is_contiguous() or p.is_conj() or p.is_neg():
+                return None
+        return base
 
     def _bwd_fused(self, f, blocks, side, length):
         B, C = blocks[0].shape[:2]

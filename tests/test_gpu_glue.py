@@ -233,3 +233,26 @@ def test_both_paths_launch_one_direction_at_a_time(cqt):
     with ThreadPoolExecutor(8) as pool:
         got = list(pool.map(lambda i: (t, twin)[i % 2].bwd(*(t, twin)[i // 2 % 2].fwd(xs[i % 4])), range(64)))
     assert all(torch.equal(y, want[i % 4]) for i, y in enumerate(got))
+
+
+def test_sliced_inverse_of_turned_and_cropped_views():
+    """bwd reads fwd's buffer in place for all of its blocks alone: the C++ check
+    and the Python one answer alike."""
+    from flash_cqt import SlicedCQT
+    sliced = SlicedCQT(fs=44100, device="cuda:0")
+    x = torch.randn(3, 1, 70001, generator=torch.Generator(device="cuda").manual_seed(4), device="cuda")
+    f = sliced.cqt.f
+    with torch.no_grad():
+        blocks, side = sliced.fwd(x)
+        parts, rows = [*blocks, *side], 3 * sliced._num_slices(70001)
+        own = [c.clone() for c in parts]
+        assert f._glue.block_base(parts, rows).data_ptr() == parts[0].data_ptr()
+        assert sliced._block_base(f, parts, rows).data_ptr() == parts[0].data_ptr()
+        first = [parts[0][:2], *parts[1:]]
+        for bad in (own, [c.conj() for c in parts], [*parts[:-1], parts[-1].conj()], [parts[1], parts[0], *parts[2:]],
+                    first, [*parts[:-1], parts[-1][:2]], parts[:-1], [*parts, parts[0]], [c[1:] for c in parts]):
+            assert f._glue.block_base(bad, rows) is None and sliced._block_base(f, bad, rows) is None
+        ng = len(blocks)
+        assert torch.equal(sliced.bwd(parts[:ng], parts[ng:]), sliced.bwd(own[:ng], own[ng:]))
+        tail = [c[1:] for c in parts]
+        assert torch.equal(sliced.bwd(tail[:ng], tail[ng:]), sliced.bwd(own[:ng], own[ng:])[1:])

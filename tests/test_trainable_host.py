@@ -149,3 +149,21 @@ def test_failed_glue_build_leaves_none_behind(monkeypatch, tmp_path):
     with pytest.raises(RuntimeError, match="glue"):
         b.build()
     assert not old.exists()
+
+
+def test_sliced_part_of_the_views_is_not_the_buffer():
+    """A block cropped to fewer signals, or blocks left out: refused, as blocks of
+    their own are, or taken as zero, not completed from the buffer."""
+    import types
+    from flash_cqt.sliced import SlicedCQT
+    s = SlicedCQT.__new__(SlicedCQT)
+    f = types.SimpleNamespace(gspec=GSPEC, ncoef=NCOEF, dev=torch.device("cpu"))
+    coef = _kc(6).flatten().clone()
+    views = [coef[6 * off:6 * (off + b * M)].view(3, 1, b, 2 * M) for b, M, off in GSPEC]
+    assert s._block_buffer(f, views[:2], views[2:], 3, 2) is coef
+    for i in range(1, 3):
+        cut = [c[:2] if j == i else c for j, c in enumerate(views)]
+        with pytest.raises(RuntimeError):
+            s._block_buffer(f, cut[:2], cut[2:], 3, 2)
+    got = s._block_buffer(f, views[:2], [], 3, 2)
+    assert torch.equal(got[:96], coef[:96]) and not got[96:].any()
