@@ -217,8 +217,8 @@ py::object fwd(const Ref& e, const Tensor& x) {
 }
 
 // The [B, ncoef] buffer whose consecutive group views the parts are, else an undefined tensor.
-// A part that is a leaf of its own, or whose gradient is wanted where the buffer's is not, is no
-// such view: its gradient would go past it.
+// A part that is a leaf of its own, that keeps its gradient or has hooks on it, or whose gradient is
+// wanted where the buffer's is not, is no such view: its gradient would go past it.
 Tensor base_of(const Engine& e, const std::vector<Tensor>& parts, int64_t batch) {
     if (!parts[0].is_view()) return {};
     const Tensor base(parts[0]._base());
@@ -231,7 +231,10 @@ Tensor base_of(const Engine& e, const std::vector<Tensor>& parts, int64_t batch)
     for (size_t i = 0; i < parts.size(); ++i) {
         const Tensor& c = parts[i];
         const Group& g = e.groups[i];
-        if (grad && (c.requires_grad() != base.requires_grad() || (c.requires_grad() && c.is_leaf()))) return {};
+        if (grad && (c.requires_grad() != base.requires_grad() ||
+                     (c.requires_grad() &&
+                      (c.is_leaf() || c.retains_grad() || !torch::autograd::impl::hooks(c).empty()))))
+            return {};
         if (!c.is_view() || !c._base().is_same(base) || static_cast<const char*>(c.data_ptr()) != ptr + 8 * g.off)
             return {};
         int64_t want = e.tab.ncoef;                    // strides of the leading dimensions, last first

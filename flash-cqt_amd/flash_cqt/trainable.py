@@ -38,20 +38,16 @@ class TrainableCQT:
 
     def _plain(self, tensors):
         """The host glue when every tensor is an ordinary one, the engine is the
-        one that the glue belongs to with the library it was attached to, and
-        the directions below are this class's own (the glue itself declines
-        what else it does not take), else None."""
+        one that the glue belongs to with the library it was attached to, and no
+        direction is replaced, by a subclass, on the class or on this object
+        (the glue would pass such a method by; what else it does not take it
+        declines itself), else None."""
         glue, f = self._glue, self.f
         if glue is not None and f._glue is glue and f.lib is self._lib and not torch.compiler.is_compiling() \
-                and all(type(t) is torch.Tensor or type(t) is torch.nn.Parameter for t in tensors) \
-                and self._own_directions():
+                and _ORDINARY.issuperset(map(type, tensors)) and _directions(type(self)) == _OWN \
+                and self.__dict__.keys().isdisjoint(_NAMES):
             return glue
         return None
-
-    def _own_directions(self):
-        """No direction replaced, by a subclass, on the class or on this object:
-        the glue would pass such a method by."""
-        return _directions(type(self)) == _OWN and self.__dict__.keys().isdisjoint(_NAMES)
 
     # ------------------------------------------------ engine directions
     # The inputs reaching these are [B, N] float32 or [B, ncoef] complex64,
@@ -125,8 +121,9 @@ class TrainableCQT:
     def _base_of(self, parts, B):
         """The [B, ncoef] complex64 buffer whose consecutive group views the
         parts are (as fwd returns them), else None. A part that is a leaf of
-        its own, or whose gradient is wanted where the buffer's is not, is no
-        such view: its gradient would go past it."""
+        its own, that keeps its gradient or has hooks on it, or whose gradient
+        is wanted where the buffer's is not, is no such view: its gradient
+        would go past it."""
         base = parts[0]._base
         if len(parts) != len(self.gspec) or base is None or base.device != self.dev or base.dtype != torch.complex64 \
                 or base.shape != (B, self.ncoef) or not base.is_contiguous():
@@ -134,7 +131,8 @@ class TrainableCQT:
         ptr = base.data_ptr()
         grad = torch.is_grad_enabled()
         for c, (b, M, off) in zip(parts, self.gspec):
-            if grad and (c.requires_grad != base.requires_grad or (c.requires_grad and c.is_leaf)):
+            if grad and (c.requires_grad != base.requires_grad
+                         or (c.requires_grad and (c.is_leaf or c.retains_grad or c._backward_hooks))):
                 return None
             if c._base is not base or c.data_ptr() != ptr + 8 * off or c.stride()[-2:] != (M, 1) \
                     or c.shape[-2:] != (b, M) or c.is_conj() or c.is_neg():
@@ -149,7 +147,12 @@ class TrainableCQT:
         return base
 
     def bwd(self, blocks, side=None):
-        """Inverse of fwd; side=None treats the DC and Nyquist bands as zero."""
+        """Inverse of fwd; side=None treats the DC and Nyquist bands as zero.
+
+        Handed fwd's own views back, it reads their buffer, and the gradient
+        goes to that buffer: torch.autograd.grad with respect to the views
+        themselves needs views that keep their gradient (retain_grad) or blocks
+        of their own (c.clone())."""
         if side is not None:
             parts = list(blocks) + list(side)
             glue = self._plain(parts)
@@ -177,6 +180,8 @@ class TrainableCQT:
             raise ValueError(f"blocks are on {flat.device}, engine on {self.dev}")
         return _Synthesis.apply(flat.resolve_conj().contiguous(), self).reshape(*lead, N)
 
+
+_ORDINARY = frozenset((torch.Tensor, torch.nn.Parameter))
 
 # the methods that the host glue stands in for
 _NAMES = ("_launch_analysis", "_launch_synthesis", "_analysis", "_synthesis", "_adj_analysis", "_adj_synthesis",

@@ -256,3 +256,26 @@ def test_sliced_inverse_of_turned_and_cropped_views():
         assert torch.equal(sliced.bwd(parts[:ng], parts[ng:]), sliced.bwd(own[:ng], own[ng:]))
         tail = [c[1:] for c in parts]
         assert torch.equal(sliced.bwd(tail[:ng], tail[ng:]), sliced.bwd(own[:ng], own[ng:])[1:])
+
+
+@pytest.mark.parametrize("path", ["glue", "python"])
+def test_watched_blocks_see_their_gradients(cqt, path):
+    """Blocks that keep their gradient, or have a hook, between fwd and bwd."""
+    t = _engine(cqt, path)
+    seen = []
+
+    def gradients(watched):
+        x = _x(3).requires_grad_(True)
+        blocks, side = t.fwd(x)
+        if watched:
+            blocks[2].retain_grad()
+            blocks[4].register_hook(lambda g: seen.append(g.clone()))
+            own = blocks
+        else:
+            own = [c.clone() for c in blocks]
+            own[2].retain_grad(), own[4].retain_grad()
+        y = t.bwd(own, side)
+        (y ** 3).sum().backward()
+        return [x.grad, own[2].grad] + (seen if watched else [own[4].grad])
+    got, want = gradients(True), gradients(False)
+    assert len(got) == 3 and all(g is not None and torch.allclose(g, w, rtol=1e-5, atol=1e-5 * float(w.abs().max())) for g, w in zip(got, want))

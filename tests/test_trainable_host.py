@@ -167,3 +167,12 @@ def test_sliced_part_of_the_views_is_not_the_buffer():
             s._block_buffer(f, cut[:2], cut[2:], 3, 2)
     got = s._block_buffer(f, views[:2], [], 3, 2)
     assert torch.equal(got[:96], coef[:96]) and not got[96:].any()
+
+
+@pytest.mark.parametrize("watch", [lambda c: c.retain_grad(), lambda c: c.register_hook(lambda g: g)])
+def test_watched_views_are_not_the_buffer(engine, watch):
+    kc = _kc().requires_grad_(True) * 1
+    parts = _views(kc, 6)
+    assert engine._base_of(parts, 6) is kc
+    watch(parts[1])
+    assert engine._base_of(parts, 6) is None
